@@ -90,7 +90,7 @@ GenericModel* buildGenericModel(int nj, const int* parents, const int* types) {
     r[GJ_NCHILD] = nchild[j];
     g->nvlev = std::max(g->nvlev, r[GJ_DOFLEVEL] + nvj[j]);
   }
-  // one device buffer: ev | jr | colPtr | patRow | nzMask
+  // one device buffer: ev | jr | colPtr | patRow | nzMask | tree-parallel tables
   std::vector<int32_t> tab;
   const size_t oEv = tab.size();
   tab.insert(tab.end(), ev.begin(), ev.end());
@@ -103,6 +103,7 @@ GenericModel* buildGenericModel(int nj, const int* parents, const int* types) {
   const size_t oNz = tab.size();
   for (uint32_t w : nz) tab.push_back((int32_t)w);
   tab.push_back(0);  // keeps every sub-table non-empty
+  g->tree.reset(buildTreeProgram(nj, parents, types, tab));
   HIP_CHECK(hipMalloc(&g->dtab, tab.size() * sizeof(int32_t)));
   HIP_CHECK(hipMemcpy(g->dtab, tab.data(), tab.size() * sizeof(int32_t), hipMemcpyHostToDevice));
   g->ev = g->dtab + oEv;
@@ -110,6 +111,7 @@ GenericModel* buildGenericModel(int nj, const int* parents, const int* types) {
   g->colPtr = g->dtab + oCp;
   g->patRow = g->dtab + oPr;
   g->nzMask = reinterpret_cast<const uint32_t*>(g->dtab + oNz);
+  if (g->tree) g->tree->place(g->dtab);
   return g.release();
 }
 

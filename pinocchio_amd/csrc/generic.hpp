@@ -5,9 +5,11 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <memory>
 #include <vector>
 
 #include "ops.hpp"
+#include "tree.hpp"
 
 namespace rbd {
 
@@ -30,6 +32,9 @@ struct GenericModel {
   mutable size_t laneBytes = 0;
   mutable std::vector<void*> retired;
   void* laneMem(size_t bytes) const;
+
+  // tables of the tree-parallel kernels; null when the numbering is not depth first
+  std::unique_ptr<TreeProgram> tree;
 
   GenericModel() = default;
   GenericModel(const GenericModel&) = delete;

@@ -229,6 +229,19 @@ int vec3Op(rbd_ctx* ctx, const rbd_model* m, int64_t B, const void* x0, int64_t 
   });
 }
 
+// M into a dense output of either layout
+template<class S>
+void crbaInto(rbd_ctx* ctx, const rbd_model* m, int64_t B, CView<S> q, View<S> M, int upper) {
+  const S* mc;
+  if constexpr (std::is_same_v<S, float>) mc = m->mc32;
+  else mc = m->mc64;
+  if (treePays(TreeOp::kCrba, m->prebuilt && m->prebuilt->crba_f32, M.rs == 1, m->nv, sizeof(S), B) &&
+      treeCrba<S>(ctx->stream, m->gen.get(), mc, B, q, M, upper))
+    return;
+  if constexpr (std::is_same_v<S, float>) m->ops->crba_f32(ctx->stream, m->gen.get(), mc, B, q, M, upper);
+  else m->ops->crba_f64(ctx->stream, m->gen.get(), mc, B, q, M, upper);
+}
+
 }  // namespace
 
 // rnea / aba with external forces (run-time-topology kernels for every tree)
@@ -668,10 +681,10 @@ int rbd_crba(rbd_ctx* ctx, const rbd_model* m, int64_t B, int dtype, const void*
     void* dM = st.out(M, vM.extent * es, true);
     const int upper = (flags & RBD_UPPER_ONLY) ? 1 : 0;
     if (f32)
-      m->ops->crba_f32(ctx->stream, m->gen.get(), m->mc32, B, CView<float>{(const float*)dq, vq.rs, vq.bs},
-                       View<float>{(float*)dM, vM.rs, vM.bs}, upper);
+      crbaInto<float>(ctx, m, B, CView<float>{(const float*)dq, vq.rs, vq.bs}, View<float>{(float*)dM, vM.rs, vM.bs},
+                      upper);
     else
-      m->ops->crba_f64(ctx->stream, m->gen.get(), m->mc64, B, CView<double>{(const double*)dq, vq.rs, vq.bs},
+      crbaInto<double>(ctx, m, B, CView<double>{(const double*)dq, vq.rs, vq.bs},
                        View<double>{(double*)dM, vM.rs, vM.bs}, upper);
     finishCall(ctx, flags, st);
   });
@@ -981,6 +994,12 @@ int rbd_compute_minverse(rbd_ctx* ctx, const rbd_model* m, int64_t B, int dtype,
       // host outputs with gaps (padded leading dimension, batch-fastest layout) are
       // preloaded so the copy back leaves the gaps as the caller had them
       float* Mi = (float*)st.out(Minv, vo.extent * 4, (flags & RBD_LAYOUT_BATCH) || ldM != (int64_t)nv * nv);
+      if (treePays(TreeOp::kMinv, m->prebuilt && m->prebuilt->crba_f32, vo.rs == 1, nv, 4, B) &&
+          treeMinv<float>(ctx->stream, m->gen.get(), m->mc32, B, CView<float>{dq_, vq.rs, vq.bs},
+                          View<float>{Mi, vo.rs, vo.bs})) {
+        finishCall(ctx, flags, st);
+        return;
+      }
       // M into the output buffer, its FP32 tree factor into the workspace, then the unit
       // right-hand sides of the solve overwrite M with its inverse
       const size_t nU = (size_t)(nnz > 0 ? nnz : 1) * B, nD = (size_t)nv * B;
@@ -1001,6 +1020,12 @@ int rbd_compute_minverse(rbd_ctx* ctx, const rbd_model* m, int64_t B, int dtype,
     Staged st{ctx, (flags & RBD_HOST_PTRS) != 0};
     const double* dq_ = (const double*)st.in(q, vq.extent * 8);
     double* Mi = (double*)st.out(Minv, vo.extent * 8, (flags & RBD_LAYOUT_BATCH) || ldM != (int64_t)nv * nv);
+    if (treePays(TreeOp::kMinv, m->prebuilt && m->prebuilt->crba_f32, vo.rs == 1, nv, 8, B) &&
+        treeMinv<double>(ctx->stream, m->gen.get(), m->mc64, B, CView<double>{dq_, vq.rs, vq.bs},
+                         View<double>{Mi, vo.rs, vo.bs})) {
+      finishCall(ctx, flags, st);
+      return;
+    }
     const size_t nU = (size_t)(nnz > 0 ? nnz : 1) * B, nD = (size_t)nv * B;
     double* wU = (double*)ctx->workspace((nU + nD) * 8);
     double* wD = wU + nU;

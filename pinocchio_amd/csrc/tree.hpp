@@ -1,0 +1,39 @@
+// tree.hpp -- launchers of the tree-parallel kernels (k_tree.hpp).  Host side; internal.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <memory>
+#include <vector>
+
+#include "ops.hpp"
+
+namespace rbd {
+
+struct TProg;
+
+// Tables of one model's tree for the tree-parallel kernels: `word` is where they start in
+// the model's table buffer, place() is told its device address.
+struct TreeProgram {
+  size_t word = 0;
+  std::unique_ptr<TProg> g;
+  void place(const int32_t* dev);
+  TreeProgram();
+  TreeProgram(const TreeProgram&) = delete;
+  TreeProgram& operator=(const TreeProgram&) = delete;
+  ~TreeProgram();
+};
+TreeProgram* buildTreeProgram(int nj, const int* parents, const int* types, std::vector<int32_t>& words);
+
+// Whether a call is faster on the tree-parallel kernels.  prebuilt: the tree has kernels of
+// its own; rows: the output keeps a configuration's elements together (rs == 1); es: bytes
+// of a scalar.
+enum class TreeOp { kCrba, kMinv };
+bool treePays(TreeOp op, bool prebuilt, bool rows, int nv, int es, int64_t B);
+
+// Each returns false, having launched nothing, when the model has no tree program or its
+// state does not fit the LDS: the caller then runs the lane-per-configuration kernels.
+template<class S> bool treeCrba(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, View<S> M, int upper);
+template<class S> bool treeMinv(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, View<S> X);
+
+}  // namespace rbd

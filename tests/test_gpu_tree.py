@@ -1,0 +1,85 @@
+"""Tree-parallel kernels against the FP64 oracle at the sizes where their tiles of eight
+configurations, levels and rounds can go wrong, on every route of the dispatch (prebuilt
+and run-time topologies, both layouts and precisions, padded leading dimensions).
+
+Bars (per configuration, infinity norm, relative): FP32 sums over a tree of at most 40
+joints as the other kernels' tests (M 1e-5; products with M^-1 4e-4, its conditioning);
+FP64 1e-12 and 1e-9.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle
+import pinocchio_amd as pa
+from helpers import f32_round, inputs, rel_err_mats
+from pinocchio_amd import models as M
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+TREES = [M.manipulator6, M.quadruped18, M.humanoid36, M.free_body, M.pendulum,
+         lambda: M.random_tree(27, 41), lambda: M.random_tree(20, 7, free_flyer=False),
+         lambda: M.serial_chain(30, 3)]
+BATCHES = [1, 7, 8, 9, 200]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    return pa.Context(0)
+
+
+def _inputs(d, B, dt):
+    x = inputs(d, B)
+    return f32_round(*x) if dt == torch.float32 else x
+
+
+def _dev(x, layout, dt):
+    return torch.tensor(np.ascontiguousarray(x.T if layout == "col" else x), dtype=dt, device="cuda")
+
+
+@pytest.mark.parametrize("tree", range(len(TREES)))
+@pytest.mark.parametrize("dt,bar,bar_inv", [(torch.float32, 1e-5, 4e-4), (torch.float64, 1e-12, 1e-9)])
+def test_crba_and_minverse(ctx, tree, dt, bar, bar_inv):
+    d = TREES[tree]()
+    for runtime in (False, True):
+        m = pa.Model(ctx, d, runtime_topology=runtime)
+        for B in BATCHES:
+            q = _inputs(d, B, dt)[0]
+            ref = oracle.crba(d, q)
+            inv = np.linalg.inv(ref)
+            up = np.triu(ref)
+            if d.jtype[1] == M.JT_FREEFLYER:  # upper-only keeps a joint's own block full
+                up[:, :6, :6] = ref[:, :6, :6]
+            for layout in ("col", "batch"):
+                e = pa.Engine(m, layout)
+                x = _dev(q, layout, dt)
+                num = lambda t: e.mats_to_numpy(t, layout, d.nv)  # noqa: E731
+                assert rel_err_mats(num(e.crba(x)), ref).max() < bar, (d.name, B, layout)
+                assert rel_err_mats(num(e.crba(x, upper_only=True)), up).max() < bar, (d.name, B, layout)
+                assert rel_err_mats(num(e.compute_minverse(x)), inv).max() < bar_inv, (d.name, B, layout)
+
+
+@pytest.mark.parametrize("pad", [1, 3, 4])
+def test_crba_padded_leading_dimension(ctx, pad):
+    """Rows that are not 16-byte aligned, and gaps that stay as the caller had them."""
+    d = M.humanoid36()
+    m = pa.Model(ctx, d)
+    B, nv = 83, d.nv
+    q = f32_round(inputs(d, B)[0])[0]
+    ref = oracle.crba(d, q)
+    for layout, shape in (("col", (B, nv * nv + pad)), ("batch", (nv * nv, B + pad))):
+        x = _dev(q, layout, torch.float32)
+        out = torch.full(shape, 7.0, dtype=torch.float32, device="cuda")
+        flags = pa.RBD_LAYOUT_BATCH if layout == "batch" else 0
+        ld = out.stride(0)
+        pa._check(pa.lib().rbd_crba(ctx.handle, m.handle, pa._i64(B), pa.RBD_F32, pa._ptr(x), pa._i64(x.stride(0)),
+                                    pa._ptr(out), pa._i64(ld), ctypes.c_uint32(flags)))
+        o = out.double().cpu().numpy()
+        if layout == "col":
+            got, gap = o[:, :nv * nv].reshape(B, nv, nv).transpose(0, 2, 1), o[:, nv * nv:]
+        else:
+            got, gap = o[:, :B].reshape(nv, nv, B).transpose(2, 1, 0), o[:, B:]
+        assert rel_err_mats(got, ref).max() < 1e-5
+        assert (gap == 7.0).all()
