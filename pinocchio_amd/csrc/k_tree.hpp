@@ -35,9 +35,12 @@ struct TProg {
   int oSubJ;              // per joint: joints of its subtree
   int oDofJ, oDl, oRp, oSub;  // per dof: joint, number of ancestor dofs, rp, subtree dofs
   int oCp, oPat;          // ancestors a of dof c, root first: pairs (a, rp[a]) from pat[2 cp[c]]
-  int oLvl, oItems;       // treeFactor: per dof level the first and first W item; the items
+  int oLvl, oItems;       // treeFactor: first item of each phase by segment level; the items
+  int oFSeg, nslev;       // its segments (first dof, length) and their levels
+  int oPairs;             // (r | c << 8) of the entries with r <= c; read from memory
+  int oSeg, nseg;         // chain segments: first dof and length (up to four consecutive dofs)
   int oCommon;            // bytes, nv x nv: number of common strict ancestors of r and c
-  int nj, nq, nv, nlog, nvlev, nnz;
+  int nj, nq, nv, nlog, nnz;
   uint32_t nvMagic;       // ceil(2^32 / nv): e / nv by multiplication for e < 2^16
 };
 enum : int { TJ_PARENT = 0, TJ_TYPE, TJ_IQ, TJ_IV, TJ_NV, TJ_REC };
@@ -310,23 +313,23 @@ __global__ __launch_bounds__(kTreeMaxThreads) void t_crba(TProg g, const S* __re
 
 // ---------------------------------------------------------------------------------------
 // Tree factorisation M = U D U^T of the packed LDS copy (cholesky.hxx:17-62) and W = U^-1
-// (same packing: the inverse of a tree factor keeps its pattern), by dof level from the
-// deepest up.  For a dof j of the level and an ancestor-or-self r (left-looking),
-//   A[r][j] = M[r][j] - sum_{k below j} A[r][k] A[j][k] / D[k]       (k = j + 1 .. j + sub[j] - 1),
-// and for a dof r of the level and a dof k below it, with the path dofs m between them,
-//   W[r][k] = -(A[r][k] / D[k] + sum_m A[r][m] / D[m] W[m][k]).
-// Both read deeper levels only, so a level is one phase; where its items are few (the
-// trunk, whose sums are long) two or four workers share a sum.  With W explicit, M^-1 =
-// W^T D^-1 W and a product with it is a sum over ancestors or descendants without a chain
-// from row to row (the triangular sweeps, 36 dependent rows, took 40 us on the humanoid;
-// factor and W in two sweeps of levels 29 us).  Leaves D on sM's diagonal, 1 / D in sDi.
-// Items: rp[r], rp[j], j, sub[j];  rp[r], k, first path entry, path length.
+// (same packing: the inverse of a tree factor keeps its pattern).  Dofs are eliminated in
+// segments S of up to four consecutive dofs of a chain that branches at its end only, the
+// segments of one level of the tree of segments together, from the deepest up:
+//   1  A[r][c] -= sum_k A[r][k] A[c][k] / D[k]   rows r above or in S, columns c of S, k below S;
+//   2  S itself, in the registers of every row's worker: its own entries of A stay as they
+//      are in LDS, its D and W_SS are written by one worker;
+//   3  W[S][k] = -W_SS (A[S][k] / D[k] + sum_m A[S][m] / D[m] W[m][k])   k below S, m between.
+// 3 of a level reads nothing that 1 of the next writes: one phase.  With W explicit, M^-1 =
+// W^T D^-1 W is a sum over ancestors without a chain from row to row.  One level per dof
+// instead of per segment (three times the phases, one column per item) took 21 us of a
+// tile, triangular sweeps with U 40 us, against 9.
+// Leaves 1 / D in sDi and W in sW.
 // ---------------------------------------------------------------------------------------
 struct __align__(8) TItem {
-  int16_t a, b, c, d;
-};
-// sum over the 2^sh (1, 2 or 4) neighbouring workers of a wave
-template<class S> __device__ __forceinline__ S treePartSum(S x, int sh) {
+  int16_t a, b, c, d;  // 1: rp[r], r, segment, row in S (-1: above);  2: rp[r], segment, -, S itself
+};                     // 3: k, segment, first path entry, path length
+template<class S> __device__ __forceinline__ S treePartSum(S x, int sh) {  // over 2^sh workers
   const S y = x + __shfl_xor(x, kTreeT);
   x = sh > 0 ? y : x;
   const S z = x + __shfl_xor(x, 2 * kTreeT);
@@ -334,12 +337,23 @@ template<class S> __device__ __forceinline__ S treePartSum(S x, int sh) {
 }
 template<class S>
 __device__ __forceinline__ void treeFactor(const TProg& g, const int16_t* tb, S* sM, S* sDi, S* sW) {
-  const int b = treeB(), w = treeW(), NW = treeNW();
+  const int b = treeB(), w = treeW(), NW = treeNW(), nnz = g.nnz;
   const TItem* items = reinterpret_cast<const TItem*>(tb + g.oItems);
-  for (int l = g.nvlev - 1; l >= 0; --l) {
-    const int f0 = tb[g.oLvl + 2 * l], f1 = tb[g.oLvl + 2 * l + 1], n = tb[g.oLvl + 2 * l + 2] - f0;
-    // workers [0, nf) take the factor's items, in whole waves, the following ones W's
-    const int nF = f1 - f0, nW = n - nF;
+  S* M = sM + b;
+  S* Di = sDi + b;
+  S* W = sW + b;
+  auto cols = [&](int seg, int& c0, int& n, int (&rp)[4]) {
+    c0 = tb[g.oFSeg + 2 * seg];
+    n = tb[g.oFSeg + 2 * seg + 1];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) rp[i] = tb[g.oRp + c0 + (i < n ? i : 0)];
+  };
+  for (int l = g.nslev - 1; l >= -1; --l) {
+    // items of 1 at this level, then of 3 at the level below
+    const int16_t* lv = tb + g.oLvl + 4 * (l + 1);
+    const int f0 = lv[0], f1 = lv[1], f2 = lv[2], f3 = lv[3];
+    const int nF = f1 - f0, nW = f2 - f1;
+    // workers [0, nf) take 1, in whole waves, the following ones 3; few items: shared sums
     const int shF = nF * 8 <= NW ? 2 : (nF * 4 <= NW ? 1 : 0), nf = ((nF << shF) + 7) & ~7;
     const int shW = nf + nW * 4 <= NW ? 2 : (nf + nW * 2 <= NW ? 1 : 0), nw = nf + (nW << shW);
     for (int i0 = 0; i0 < nw; i0 += NW) {  // uniform: every lane takes part in the shuffles
@@ -348,51 +362,102 @@ __device__ __forceinline__ void treeFactor(const TProg& g, const int16_t* tb, S*
       const int sh = fac ? shF : shW, parts = 1 << sh, part = i & (parts - 1);
       const int id = fac ? i >> sh : nF + ((i - nf) >> sh);
       const bool on = fac ? id < nF : i < nw;
-      const TItem it = items[f0 + (on ? id : 0)];
-      const S* x = sM + it.a * kTreeT + b;
-      S acc = S(0), m = S(0);
-      S* dst;
-      // sums in batches of four, the last one filled up with zero weights
-      if (fac) {
-        const S* y = sM + it.b * kTreeT + b;
-        const int j = it.c, last = j + it.d - 1;
-        dst = sM + (it.a == it.b ? g.nnz + j : it.a + j) * kTreeT + b;
-        m = *dst;
-        for (int k = j + 1 + part; k <= last; k += 4 * parts) {
-          S u[4], v[4], d[4];
+      S acc[4] = {};
+      if (on) {
+        const TItem it = items[f0 + id];
+        int c0, n, rp[4];
+        cols(fac ? it.c : it.b, c0, n, rp);
+        if (fac) {
+          const S* x = M + it.a * kTreeT;
+          const int last = c0 + tb[g.oSub + c0] - 1;
+          for (int k = c0 + n + part; k <= last; k += 2 * parts) {
+            const int k2 = k + parts <= last ? k + parts : last;
+            const S u = x[k * kTreeT] * Di[k * kTreeT];
+            const S v = k + parts <= last ? x[k2 * kTreeT] * Di[k2 * kTreeT] : S(0);
 #pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            const int kk = k + t * parts <= last ? k + t * parts : last;
-            u[t] = x[kk * kTreeT];
-            v[t] = y[kk * kTreeT];
-            d[t] = sDi[kk * kTreeT + b];
-            d[t] = k + t * parts <= last ? d[t] : S(0);
+            for (int t = 0; t < 4; ++t) acc[t] += u * M[(rp[t] + k) * kTreeT] + v * M[(rp[t] + k2) * kTreeT];
           }
+        } else {
+          const int k = it.a;
+          for (int p = part; p < it.d; p += parts) {
+            const TAnc q = treeAnc(g, tb, it.c + p);
+            const S u = W[(q.rp + k) * kTreeT] * Di[q.a * kTreeT];
 #pragma unroll
-          for (int t = 0; t < 4; ++t) acc += u[t] * (v[t] * d[t]);
-        }
-      } else {
-        const int k = it.b, last = it.d - 1;
-        dst = sW + (it.a + k) * kTreeT + b;
-        m = x[k * kTreeT] * sDi[k * kTreeT + b];
-        for (int p = part; p <= last; p += 4 * parts) {
-          S u[4], v[4], d[4];
-#pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            const TAnc q = treeAnc(g, tb, it.c + (p + t * parts <= last ? p + t * parts : last));
-            u[t] = x[q.a * kTreeT];
-            v[t] = sW[(q.rp + k) * kTreeT + b];
-            d[t] = sDi[q.a * kTreeT + b];
-            d[t] = p + t * parts <= last ? d[t] : S(0);
+            for (int t = 0; t < 4; ++t) acc[t] += u * M[(rp[t] + q.a) * kTreeT];
           }
-#pragma unroll
-          for (int t = 0; t < 4; ++t) acc += u[t] * (v[t] * d[t]);
         }
       }
-      acc = treePartSum(acc, sh);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) acc[t] = treePartSum(acc[t], sh);
       if (on && part == 0) {
-        *dst = fac ? m - acc : -(m + acc);
-        if (fac && it.a == it.b) sDi[it.c * kTreeT + b] = S(1) / (m - acc);
+        const TItem it = items[f0 + id];
+        int c0, n, rp[4];
+        cols(fac ? it.c : it.b, c0, n, rp);
+        if (fac) {
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+            if (t < n && t >= it.d) M[(t == it.d ? nnz + c0 + t : it.a + c0 + t) * kTreeT] -= acc[t];
+        } else {
+          const int k = it.a;
+          const S d = Di[k * kTreeT];
+          S v[4];
+#pragma unroll
+          for (int t = 0; t < 4; ++t) v[t] = t < n ? acc[t] + M[(rp[t] + k) * kTreeT] * d : S(0);
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            S x = v[t];
+#pragma unroll
+            for (int o = t + 1; o < 4; ++o) x += o < n ? W[(rp[t] + c0 + o) * kTreeT] * v[o] : S(0);
+            if (t < n) W[(rp[t] + k) * kTreeT] = -x;
+          }
+        }
+      }
+    }
+    __syncthreads();
+    if (l < 0) break;
+    for (int i = f2 + w; i < f3; i += NW) {
+      const TItem it = items[i];
+      int c0, n, rp[4];
+      cols(it.b, c0, n, rp);
+      S a[4], s[4][4], di[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        a[c] = !it.d && c < n ? M[(it.a + c0 + c) * kTreeT] : S(0);
+        s[c][c] = c < n ? M[(nnz + c0 + c) * kTreeT] : S(1);
+#pragma unroll
+        for (int r = 0; r < c; ++r) s[r][c] = c < n ? M[(rp[r] + c0 + c) * kTreeT] : S(0);
+      }
+#pragma unroll
+      for (int c = 3; c >= 0; --c) {
+        di[c] = S(1) / s[c][c];
+#pragma unroll
+        for (int j = 0; j < c; ++j) {
+          const S u = s[j][c] * di[c];
+          a[j] -= a[c] * u;
+#pragma unroll
+          for (int r = 0; r <= j; ++r) s[r][j] -= s[r][c] * u;
+        }
+      }
+      if (!it.d) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (c < n) M[(it.a + c0 + c) * kTreeT] = a[c];
+      } else {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (c < n) Di[(c0 + c) * kTreeT] = di[c];
+        // W_SS: inverse of the unit upper block U = s / D
+        S v[4][4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+          for (int r = c - 1; r >= 0; --r) {
+            S x = s[r][c] * di[c];
+#pragma unroll
+            for (int m = r + 1; m < c; ++m) x += s[r][m] * di[m] * v[m][c];
+            v[r][c] = -x;
+            if (c < n) W[(rp[r] + c0 + c) * kTreeT] = -x;
+          }
       }
     }
     __syncthreads();
@@ -450,6 +515,297 @@ __global__ __launch_bounds__(kTreeMaxThreads) void t_minv(TProg g, const S* __re
   treeMassTile<S>(g, tb, g.nTabFactor, mc, gq, b0, nb, sW, sM);
   treeFactor<S>(g, tb, sM, sDi, sW);
   for (int e = threadIdx.x; e < g.nv * g.nv; e += blockDim.x) treePut(gX, e, treeMinvEntry<S>(g, tb, sW, sDi, e), b0, nb);
+}
+
+// ---------------------------------------------------------------------------------------
+// computeRNEADerivatives of the tile into a workspace of packed tiles, for t_dsolve: tile t
+// holds treeWsEntries entries of kTreeT configurations each,
+//   dtau_dq: upper entries (r, c), lower entries (c, r) at nnz + (r, c), diagonal; dtau_dv
+//   the same; M: upper entries, diagonal.
+// World velocities are sums of qd J over a dof's ancestors, gravity-shifted accelerations
+// sums of (parent velocity x qd J + qdd J); the composite quantities (inertia, its time
+// variation, force: 37 scalars, the variation as its symmetric-transposed block, the
+// angular block and the linear momentum that both share) are summed child into parent by
+// one worker per component; then one worker per column c emits the column's entries
+// (k_deriv.hpp).
+// LDS: kTreeRdJnt slots per joint (placements, velocity and acceleration; then the 37) and
+// kTreeRdDof per dof (J, dV/dq, dA/dq, dA/dv); two workgroups per CU on the humanoid.
+// ---------------------------------------------------------------------------------------
+constexpr int kTreeRdJnt = 37, kTreeRdDof = 25;
+inline int treeWsEntries(const TProg& g) { return 5 * g.nnz + 3 * g.nv; }
+template<class S> size_t treeRneadLds(const TProg& g) {
+  return (size_t)((g.nTab + 7) & ~7) * 2 +
+         ((size_t)g.nj * (kTreeRdJnt * kTreeT + kTreeMassC) +
+          (size_t)(g.nv * kTreeRdDof + g.nq + 2 * g.nv) * kTreeT) * sizeof(S);
+}
+template<class S>
+__global__ __launch_bounds__(kTreeMaxThreads) void t_rnead(TProg g, const S* __restrict__ mc, int64_t B, CView<S> gq,
+                                                           CView<S> gv, CView<S> ga, S* __restrict__ ws) {
+  extern __shared__ __align__(16) unsigned char t_lds[];
+  const int64_t tile = treeTile(), b0 = tile * kTreeT;
+  if (b0 >= B) return;
+  const int nb = (int)(B - b0 < kTreeT ? B - b0 : kTreeT);
+  int16_t* tb = reinterpret_cast<int16_t*>(t_lds);
+  S* sj = reinterpret_cast<S*>(tb + ((g.nTab + 7) & ~7));
+  S* sd = sj + g.nj * kTreeRdJnt * kTreeT;
+  S* sc = sd + g.nv * kTreeRdDof * kTreeT;
+  S* sq = sc + g.nj * kTreeMassC;
+  S* sv = sq + g.nq * kTreeT;
+  S* sa = sv + g.nv * kTreeT;
+  const int b = treeB(), w = treeW(), NW = treeNW();
+  auto jnt = [&](int j) { return TRec<S>{sj + j * kTreeRdJnt * kTreeT + b}; };
+  auto dof = [&](int c) { return TRec<S>{sd + c * kTreeRdDof * kTreeT + b}; };
+  treeStageTab(g, tb, g.nTab);
+  treeStageConsts<S, MC_R, 12, kTreeMassC, 0>(mc, g.nj, sc);
+  treeStageConsts<S, MC_CI, 10, kTreeMassC, 12>(mc, g.nj, sc);
+  treeStage(sq, gq, g.nq, b0, nb);
+  treeStage(sv, gv, g.nv, b0, nb);
+  treeStage(sa, ga, g.nv, b0, nb);
+  const S* __restrict__ arm = mc + g.nj * MC_REC;
+  const S* __restrict__ gr = arm + g.nv;
+  const Mot<S> a0 = {{-gr[0], -gr[1], -gr[2]}, {-gr[3], -gr[4], -gr[5]}};
+  __syncthreads();
+  const int at = treePlacements<S, kTreeRdJnt>(g, tb, sc, kTreeMassC, sq, sj, 0, 12, true);
+  // -- world axes
+  for (int c = w; c < g.nv; c += NW) {
+    const int j = tb[g.oDofJ + c], ty = tb[j * TJ_REC + TJ_TYPE], k = c - tb[j * TJ_REC + TJ_IV];
+    const Xform<S> oM = jnt(j).template get<Xform<S>>(at);
+    const int ax = ty == JT_FF ? (k < 3 ? k : k - 3) : ty - JT_RX;
+    Mot<S> J = treeWorldAxis(oM, ax);
+    if (ty == JT_FF && k < 3) J = {J.a, {S(0), S(0), S(0)}};
+    dof(c).put(0, J);
+  }
+  __syncthreads();
+  // world velocity of joint j: the sum of qd J over its last dof and that dof's ancestors
+  for (int j = 1 + w; j < g.nj; j += NW) {
+    const int c = tb[j * TJ_REC + TJ_IV] + tb[j * TJ_REC + TJ_NV] - 1, cp = tb[g.oCp + c], n = tb[g.oDl + c];
+    Mot<S> x = scale(sv[c * kTreeT + b], dof(c).template get<Mot<S>>(0));
+#pragma unroll 2
+    for (int s = 0; s < n; ++s) {
+      const int r = treeAnc(g, tb, cp + s).a;
+      x = x + scale(sv[r * kTreeT + b], dof(r).template get<Mot<S>>(0));
+    }
+    jnt(j).put(24, x);
+  }
+  __syncthreads();
+  for (int c = w; c < g.nv; c += NW) {
+    const int p = tb[tb[g.oDofJ + c] * TJ_REC + TJ_PARENT];
+    const Mot<S> J = dof(c).template get<Mot<S>>(0);
+    Mot<S> x = scale(sa[c * kTreeT + b], J);
+    if (p > 0) x = x + crossMM(jnt(p).template get<Mot<S>>(24), scale(sv[c * kTreeT + b], J));
+    dof(c).put(18, x);
+  }
+  __syncthreads();
+  for (int j = 1 + w; j < g.nj; j += NW) {
+    const int c = tb[j * TJ_REC + TJ_IV] + tb[j * TJ_REC + TJ_NV] - 1, cp = tb[g.oCp + c], n = tb[g.oDl + c];
+    Mot<S> x = a0;
+#pragma unroll 2
+    for (int s = 0; s < n; ++s) x = x + dof(treeAnc(g, tb, cp + s).a).template get<Mot<S>>(18);
+    jnt(j).put(30, x + dof(c).template get<Mot<S>>(18));
+  }
+  __syncthreads();
+  // -- column data, composite quantities of the bodies
+  for (int c = w; c < g.nv; c += NW) {
+    const int j = tb[g.oDofJ + c], p = tb[j * TJ_REC + TJ_PARENT];
+    const Mot<S> J = dof(c).template get<Mot<S>>(0), ov = jnt(j).template get<Mot<S>>(24);
+    Mot<S> dV = zeroMot<S>(), dA = crossMM(a0, J);
+    if (p > 0) {
+      const Mot<S> ovp = jnt(p).template get<Mot<S>>(24);
+      dV = crossMM(ovp, J);
+      dA = crossMM(jnt(p).template get<Mot<S>>(30), J) + crossMM(ovp, dV);
+    }
+    dof(c).put(6, dV);
+    dof(c).put(12, dA);
+    dof(c).put(18, crossMM(ov, J) + dV);
+  }
+  __syncthreads();
+  for (int j = 1 + w; j < g.nj; j += NW) {
+    const Xform<S> oM = jnt(j).template get<Xform<S>>(at);
+    const Mot<S> ov = jnt(j).template get<Mot<S>>(24), oa = jnt(j).template get<Mot<S>>(30);
+    const CInertia<S> Y = transportUp(oM, ldsConst<CInertia<S>>(sc + j * kTreeMassC + 12));
+    const Frc<S> oh = cmul(Y, ov);
+    DY<S> D = inertiaVariation(Y, ov, Frc<S>{{S(0), S(0), S(0)}, oh.a});  // LA = AL^T without oh.l
+    jnt(j).put(0, Y);
+    jnt(j).put(10, D.LA);
+    jnt(j).put(19, D.AA);
+    jnt(j).put(28, oh.l);
+    jnt(j).put(31, cmul(Y, oa) + crossMF(ov, oh));
+  }
+  __syncthreads();
+  // -- child into parent, last joint first; a chain's running sum stays in a register
+  for (int k = w; k < 37; k += NW) {
+    S* x = sj + k * kTreeT + b;
+    S cur = x[(g.nj - 1) * kTreeRdJnt * kTreeT];
+    for (int j = g.nj - 1; j > 1; --j) {
+      const int p = tb[j * TJ_REC + TJ_PARENT];
+      S next = x[(j - 1) * kTreeRdJnt * kTreeT];
+      if (p == j - 1) {
+        next += cur;
+        x[(j - 1) * kTreeRdJnt * kTreeT] = next;
+      } else if (p > 0) {
+        x[p * kTreeRdJnt * kTreeT] += cur;
+      }
+      cur = next;
+    }
+  }
+  __syncthreads();
+  // -- columns
+  const int nnz = g.nnz, nX = 2 * nnz + g.nv;
+  S* out = ws + tile * (int64_t)(5 * nnz + 3 * g.nv) * kTreeT + b;
+  auto put = [&](int e, S x) { out[e * kTreeT] = x; };
+  for (int c = w; c < g.nv; c += NW) {
+    const int j = tb[g.oDofJ + c];
+    const CInertia<S> Y = jnt(j).template get<CInertia<S>>(0);
+    const R3<S> LA0 = jnt(j).template get<R3<S>>(10);
+    const R3<S> Fl = skewM(-jnt(j).template get<V3<S>>(28));
+    const DY<S> D = {add(LA0, Fl), add(transpose(LA0), Fl), jnt(j).template get<R3<S>>(19)};
+    const Frc<S> of = jnt(j).template get<Frc<S>>(31);
+    const ColData<S> C = dof(c).template get<ColData<S>>(0);
+    const Frc<S> dFda = cmul(Y, C.J);
+    const Frc<S> dFdq = cmul(Y, C.dAdq) + dyMul(D, C.dVdq);
+    const Frc<S> dFdv = dyMul(D, C.J) + cmul(Y, C.dAdv);
+    const Frc<S> dYtJ = dyMulT(D, C.J);
+    const Frc<S> dFdqA = dFdq + crossMF(C.J, of);
+    put(2 * nnz + c, dot(C.J, dFdq));
+    put(nX + 2 * nnz + c, dot(C.J, dFdv));
+    put(2 * nX + nnz + c, dot(C.J, dFda) + arm[c]);
+    // entries below the diagonal inside a free flyer's block
+    const int c1 = tb[j * TJ_REC + TJ_IV] + tb[j * TJ_REC + TJ_NV], rpc = tb[g.oRp + c];
+    for (int c2 = c + 1; c2 < c1; ++c2) {
+      const Mot<S> J2 = dof(c2).template get<Mot<S>>(0);
+      put(nnz + rpc + c2, dot(J2, dFdq));
+      put(nX + nnz + rpc + c2, dot(J2, dFdv));
+    }
+    const int cp = tb[g.oCp + c], na = tb[g.oDl + c], own = tb[j * TJ_REC + TJ_IV];
+    for (int s = 0; s < na; ++s) {
+      const TAnc a = treeAnc(g, tb, cp + s);
+      const ColData<S> R = dof(a.a).template get<ColData<S>>(0);
+      const int e = a.rp + c;
+      const bool block = a.a >= own;  // same joint: the term J_c x* of stays out
+      put(e, block ? dot(R.J, dFdq) : dot(R.J, dFdqA));
+      put(nX + e, dot(R.J, dFdv));
+      put(2 * nX + e, dot(R.J, dFda));
+      if (!block) {
+        put(nnz + e, dot(R.dAdq, dFda) + dot(R.dVdq, dYtJ));
+        put(nX + nnz + e, dot(R.dAdv, dFda) + dot(R.J, dYtJ));
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// ABA-derivative solve on the packed tiles of t_rnead: factor of M, W = U^-1 and M^-1 in
+// LDS, then -M^-1 X for X = dtau_dq and dtau_dv.
+// Columns go four at a time: a segment of up to four consecutive dofs of one chain
+// (TProg::oSeg), so that they are zero outside the same rows, the first dof's ancestors
+// and subtree, which alone are staged and summed over.  A worker takes four rows and a
+// segment of one X: eight LDS reads for sixteen multiply-adds.  (Two sparse products with W
+// are half the multiply-adds, but two phases of short sums each: 45 us of a tile against
+// 15.)  R segments per round.
+// gridDim.y == 3, for batches whose tiles alone leave CUs idle: y = 0, 1 the even and odd
+// rounds, y = 2 M^-1 (each repeats the factor).
+// LDS: M^-1 [row][row][configuration]; the factor, over which the rounds' X goes.
+// ---------------------------------------------------------------------------------------
+__host__ __device__ __forceinline__ int treeNB(const TProg& g) { return (g.nv + 3) / 4; }  // rows ib, ib + NB, ..
+template<class S> size_t treeSolveLds(const TProg& g, int R) {
+  const size_t f = (size_t)(2 * g.nnz + 2 * g.nv) * kTreeT, x = (size_t)R * g.nv * 8 * kTreeT;
+  return (size_t)((g.nTabFactor + 7) & ~7) * 2 +
+         ((size_t)g.nv * treeNB(g) * 4 * kTreeT + (f > x ? f : x)) * sizeof(S);
+}
+template<class S>
+__global__ __launch_bounds__(kTreeMaxThreads) void t_dsolve(TProg g, int64_t B, const S* __restrict__ ws, View<S> gXq,
+                                                            View<S> gXv, View<S> gMinv, int R) {
+  extern __shared__ __align__(16) unsigned char t_lds[];
+  const int64_t tile = treeTile(), b0 = tile * kTreeT;
+  if (b0 >= B) return;
+  const int nb = (int)(B - b0 < kTreeT ? B - b0 : kTreeT);
+  const int nnz = g.nnz, nv = g.nv, nX = 2 * nnz + nv, NB = treeNB(g), PP = NB * 4 * kTreeT;
+  int16_t* tb = reinterpret_cast<int16_t*>(t_lds);
+  S* sP = reinterpret_cast<S*>(tb + ((g.nTabFactor + 7) & ~7));
+  S* sM = sP + nv * PP;
+  S* sDi = sM + (nnz + nv) * kTreeT;
+  S* sW = sDi + nv * kTreeT;
+  S* sx = sM;
+  const int b = treeB(), w = treeW(), NW = treeNW();
+  const S* in = ws + tile * (int64_t)(5 * nnz + 3 * nv) * kTreeT;
+  // -- stage M
+  treeStageTab(g, tb, g.nTabFactor);
+  for (int e = threadIdx.x; e < (nnz + nv) * kTreeT; e += blockDim.x) sM[e] = in[2 * nX * kTreeT + e];
+  __syncthreads();
+  // -- factor
+  treeFactor<S>(g, tb, sM, sDi, sW);
+  // -- inverse
+  const bool all = gridDim.y == 1;
+  for (int i = threadIdx.x; i < nv * (nv + 1) / 2; i += blockDim.x) {
+    const uint32_t rc = reinterpret_cast<const uint16_t*>(g.tab + g.oPairs)[i];
+    const int r = rc & 255, c = rc >> 8;
+    const TreeRow<S> x = treeMinvEntry<S>(g, tb, sW, sDi, c * nv + r);
+    *reinterpret_cast<TreeRow<S>*>(sP + r * PP + c * kTreeT) = x;
+    *reinterpret_cast<TreeRow<S>*>(sP + c * PP + r * kTreeT) = x;
+  }
+  __syncthreads();
+  if (all || blockIdx.y == 2) {
+    for (int e = threadIdx.x; e < nv * nv; e += blockDim.x) {
+      const int c = __umulhi(e, g.nvMagic), r = e - c * nv;
+      treePut(gMinv, e, treeRow(sP + c * PP + r * kTreeT), b0, nb);
+    }
+    if (!all) return;
+  }
+  // -- products
+  const int step = all ? R : 2 * R;
+  for (int s0 = all ? 0 : (int)blockIdx.y * R; s0 < g.nseg; s0 += step) {
+    const int ns = g.nseg - s0 < R ? g.nseg - s0 : R;
+    // X on the related rows: sx[segment][row][X][column][configuration]
+    for (int k = 0; k < ns; ++k) {
+      const int c0 = tb[g.oSeg + 2 * (s0 + k)], n = tb[g.oSeg + 2 * (s0 + k) + 1];
+      const int dl = tb[g.oDl + c0], cp = tb[g.oCp + c0], nr = dl + tb[g.oSub + c0];
+      for (int i = w; i < nr * 8; i += NW) {
+        const int idx = i >> 3, m = i & 7, col = m & 3;
+        const int r = idx < dl ? treeAnc(g, tb, cp + idx).a : c0 + idx - dl;
+        const int c = c0 + (col < n ? col : 0);
+        const int lo = r < c ? r : c, hi = r < c ? c : r;
+        const int e = lo == hi ? 2 * nnz + lo : (r < c ? 0 : nnz) + tb[g.oRp + lo] + hi;
+        sx[((k * nv + idx) * 8 + m) * kTreeT + b] =
+            hi < lo + tb[g.oSub + lo] ? in[((m >> 2) * nX + e) * kTreeT + b] : S(0);
+      }
+    }
+    __syncthreads();
+    for (int i = w; i < 2 * ns * NB; i += NW) {
+      const int kh = i / NB, ib = i - kh * NB, k = kh >> 1, h = kh & 1;
+      const int c0 = tb[g.oSeg + 2 * (s0 + k)], n = tb[g.oSeg + 2 * (s0 + k) + 1];
+      const int dl = tb[g.oDl + c0], cp = tb[g.oCp + c0], sub = tb[g.oSub + c0];
+      const S* x = sx + (k * nv * 8 + h * 4) * kTreeT + b;
+      const S* P = sP + ib * kTreeT + b;
+      S z[4][4] = {};
+      auto add = [&](const S* p) {
+        S u[4], y[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) u[t] = p[t * NB * kTreeT];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) y[t] = x[t * kTreeT];
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int o = 0; o < 4; ++o) z[t][o] -= u[t] * y[o];
+        x += 8 * kTreeT;
+      };
+#pragma unroll 2
+      for (int p = 0; p < dl; ++p) add(P + treeAnc(g, tb, cp + p).a * PP);
+#pragma unroll 2
+      for (int p = 0; p < sub; ++p) add(P + (c0 + p) * PP);
+      const View<S> out = h ? gXv : gXq;
+      S* dst = out.p + (b0 + b) * out.bs;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int o = 0; o < 4; ++o) {
+          const int r = ib + t * NB;
+          if (b < nb && r < nv && o < n) dst[(int64_t)((c0 + o) * nv + r) * out.rs] = z[t][o];
+        }
+    }
+    __syncthreads();
+  }
+  // -- end
 }
 
 }  // namespace rbd

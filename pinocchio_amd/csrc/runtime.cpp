@@ -229,6 +229,10 @@ int vec3Op(rbd_ctx* ctx, const rbd_model* m, int64_t B, const void* x0, int64_t 
   });
 }
 
+// packed tiles of the tree-parallel derivative path at a time: bounds its workspace and
+// leaves the tiles between its two kernels in the last-level cache
+constexpr size_t kTreeWsBytes = size_t(128) << 20;
+
 // M into a dense output of either layout
 template<class S>
 void crbaInto(rbd_ctx* ctx, const rbd_model* m, int64_t B, CView<S> q, View<S> M, int upper) {
@@ -892,9 +896,19 @@ void abaDerivCall(rbd_ctx* ctx, const rbd_model* m, int64_t B, const void* q, in
                                 " bytes of scratch, more than the " + std::to_string(fixedWsElems * sizeof(S)) +
                                 " available (at most " + std::to_string(fixedWsElems / (nnz + 2 * nv)) +
                                 " configurations of this model)");
-  S* wU = fixedWs ? fixedWs : (S*)ctx->workspace(need * sizeof(S));
+  // tree-parallel path: ddq, then the packed tiles of a chunk of the batch (kTreeWsBytes, or
+  // what a fixed workspace holds, bounds them); not taken in a capture for which only the
+  // other path's smaller workspace was reserved
+  const size_t te = treeDerivEntries(m->gen.get()), wsElems = fixedWs ? fixedWsElems - (size_t)nv * B
+                                                                      : kTreeWsBytes / sizeof(S);
+  const int64_t chunk = te ? std::min<int64_t>((B + 7) & ~int64_t(7), (wsElems / te) & ~size_t(7)) : 0;
+  const size_t tneed = (size_t)nv * B + te * chunk;
+  bool tree = chunk > 0 && treePays(TreeOp::kDeriv, m->prebuilt && m->prebuilt->abad_solve_f32, vo.rs == 1, nv,
+                                    sizeof(S), B);
+  if (tree && ctx->capturing && !fixedWs && ctx->workBytes < tneed * sizeof(S)) tree = false;
+  S* wU = fixedWs ? fixedWs : (S*)ctx->workspace((tree ? std::max(need, tneed) : need) * sizeof(S));
   S* wD = wU + nU;
-  S* wA = wD + nD;
+  S* wA = tree ? wU : wD + nD;
   View<S> vddq{wA, B, 1};
   if (ddq) {
     S* dd = (S*)st.out(ddq, va.extent * sizeof(S), true);
@@ -905,6 +919,23 @@ void abaDerivCall(rbd_ctx* ctx, const rbd_model* m, int64_t B, const void* q, in
   // 1. ddq = aba(q, v, tau)
   if constexpr (f32) o.aba_f32(ctx->stream, m->gen.get(), m->mc32, B, cq, cv, CView<S>{dt_, vt.rs, vt.bs}, vddq);
   else o.aba_f64(ctx->stream, m->gen.get(), m->mc64, B, cq, cv, CView<S>{dt_, vt.rs, vt.bs}, vddq);
+  if (tree) {
+    bool done = true;
+    for (int64_t c0 = 0; c0 < B && done; c0 += chunk) {
+      const int64_t n = std::min(chunk, B - c0);
+      auto at = [&](auto x) {
+        x.p += c0 * x.bs;
+        return x;
+      };
+      done = treeAbaDeriv<S>(ctx->stream, m->gen.get(), mcOf<S>(m), n, at(cq), at(cv),
+                             at(CView<S>{vddq.p, vddq.rs, vddq.bs}), at(View<S>{Xq, vo.rs, vo.bs}),
+                             at(View<S>{Xv, vo.rs, vo.bs}), at(View<S>{Mi, vo.rs, vo.bs}), wU + (size_t)nv * B);
+    }
+    if (done) {
+      finishCall(ctx, flags, st);
+      return;
+    }
+  }
   // 2. dtau_dq, dtau_dv, M at a = ddq, into the output buffers
   rneadOf<S>(m)(ctx->stream, m->gen.get(), mcOf<S>(m), B, cq, cv, CView<S>{vddq.p, vddq.rs, vddq.bs},
                 View<S>{Xq, vo.rs, vo.bs}, View<S>{Xv, vo.rs, vo.bs}, View<S>{Mi, vo.rs, vo.bs}, 7, 0);

@@ -45,7 +45,6 @@ TreeProgram* buildTreeProgram(int nj, const int* parents, const int* types, std:
       }
       dofJ[c] = j;
       dl[c] = (int)anc[c].size();
-      g.nvlev = std::max(g.nvlev, dl[c] + 1);
       cp[c + 1] = cp[c] + dl[c];
       for (int r : anc[c]) sub[r] += 1;
     }
@@ -82,25 +81,62 @@ TreeProgram* buildTreeProgram(int nj, const int* parents, const int* types, std:
   while (tab.size() & 1) tab.push_back(0);
   g.oPat = flat(pat);
   g.nTab = (int)tab.size();
-  // items by dof level (8-byte records): column entries of the factorisation, then W
-  std::vector<int> lvl, items;
-  for (int l = 0; l < g.nvlev; ++l) {
-    lvl.push_back((int)items.size() / 4);
-    for (int j = 0; j < nv; ++j)
-      if (dl[j] == l) {
-        items.insert(items.end(), {rp[j], rp[j], j, sub[j]});
-        for (int r : anc[j]) items.insert(items.end(), {rp[r], rp[j], j, sub[j]});
-      }
-    lvl.push_back((int)items.size() / 4);
-    for (int r = 0; r < nv; ++r)
-      if (dl[r] == l)
-        for (int k = r + 1; k < r + sub[r]; ++k)
-          items.insert(items.end(), {rp[r], k, cp[k] + l + 1, dl[k] - 1 - l});
+  // segments of treeFactor: a dof joins its predecessor's while that has no other child
+  std::vector<int> nkid(nv, 0), seg, segOf(nv), slev;
+  for (int c = 0; c < nv; ++c)
+    if (!anc[c].empty()) nkid[anc[c].back()] += 1;
+  for (int c = 0; c < nv; ++c) {
+    const int p = anc[c].empty() ? -1 : anc[c].back();
+    if (p >= 0 && p == c - 1 && nkid[p] == 1 && seg.back() < 4) {
+      seg.back() += 1;
+      segOf[c] = segOf[p];
+    } else {
+      segOf[c] = (int)seg.size() / 2;
+      seg.insert(seg.end(), {c, 1});
+      slev.push_back(p < 0 ? 0 : slev[segOf[p]] + 1);
+      g.nslev = std::max(g.nslev, slev.back() + 1);
+    }
   }
-  lvl.push_back((int)items.size() / 4);
+  // its items (8-byte records): phase 1 of a level with phase 3 of the level below, phase 2;
+  // level -1 (only the last phase 3) first in the table of starts
+  std::vector<int> lvl(4 * (g.nslev + 1)), items;
+  for (int l = g.nslev - 1; l >= -1; --l) {
+    int* at = &lvl[4 * (l + 1)];
+    at[0] = (int)items.size() / 4;
+    for (int s = 0; s < (int)slev.size(); ++s) {
+      const int c0 = seg[2 * s], n = seg[2 * s + 1];
+      if (slev[s] != l || sub[c0] == n) continue;  // nothing below: nothing to add
+      for (int r : anc[c0]) items.insert(items.end(), {rp[r], r, s, -1});
+      for (int i = 0; i < n; ++i) items.insert(items.end(), {rp[c0 + i], c0 + i, s, i});
+    }
+    at[1] = (int)items.size() / 4;
+    for (int s = 0; s < (int)slev.size(); ++s) {
+      const int c0 = seg[2 * s], n = seg[2 * s + 1];
+      if (slev[s] != l + 1) continue;
+      for (int k = c0 + n; k < c0 + sub[c0]; ++k)
+        items.insert(items.end(), {k, s, cp[k] + dl[c0] + n, dl[k] - dl[c0] - n});
+    }
+    at[2] = (int)items.size() / 4;
+    for (int s = 0; s < (int)slev.size(); ++s)
+      if (slev[s] == l) {
+        for (int r : anc[seg[2 * s]]) items.insert(items.end(), {rp[r], s, 0, 0});
+        items.insert(items.end(), {0, s, 0, 1});
+      }
+    at[3] = (int)items.size() / 4;
+  }
+  g.oFSeg = flat(seg);
   g.oLvl = flat(lvl);
   while (tab.size() & 3) tab.push_back(0);
   g.oItems = flat(items);
+  std::vector<int> segs;
+  for (int c = 0; c < nv;) {
+    int n = 1;
+    while (n < 4 && c + n < nv && !anc[c + n].empty() && anc[c + n].back() == c + n - 1) ++n;
+    segs.insert(segs.end(), {c, n});
+    c += n;
+  }
+  g.oSeg = flat(segs);
+  g.nseg = (int)segs.size() / 2;
   // common strict ancestors of each pair of dofs
   std::vector<uint8_t> com((size_t)nv * nv + 1);
   for (int c = 0; c < nv; ++c)
@@ -112,6 +148,9 @@ TreeProgram* buildTreeProgram(int nj, const int* parents, const int* types, std:
   g.oCommon = (int)tab.size();
   for (size_t k = 0; k + 1 < com.size(); k += 2) tab.push_back((int16_t)(com[k] | com[k + 1] << 8));
   g.nTabFactor = (int)tab.size();
+  g.oPairs = (int)tab.size();
+  for (int c = 0; c < nv; ++c)
+    for (int r = 0; r <= c; ++r) tab.push_back((int16_t)(r | c << 8));
   while (tab.size() & 3) tab.push_back(0);
   while (words.size() & 3) words.push_back(0);
   auto t = std::make_unique<TreeProgram>();
@@ -157,22 +196,27 @@ const TProg* prog(GM m) { return m->tree ? m->tree->g.get() : nullptr; }
 
 // Measured on an MI355X, us per synchronous call, lane per configuration / tree-parallel.
 // Trees without kernels of their own: faster at every size (27 joints, CRBA 232 / 22 at one
-// configuration, 1009 / 52 at 16,384 by rows, 494 / 178 at 65,536 batch-fastest; Minv 884 /
-// 42, 2118 / 155, 2749 / 513).
-// Output by rows: 36 dofs 53 / 23 at one configuration, 1078 / 58 at 16,384, 4346 / 187 at
-// 65,536 (Minv 103 / 49, 2144 / 202, 8778 / 704).  Matrices of a few hundred bytes stay
-// where they were: one configuration is a few cache lines and the serial walk is short (6
-// dofs: equal up to 16,384, FP64 21 / 28 there).
+// configuration, 1009 / 49 at 16,384 by rows, 494 / 169 at 65,536 batch-fastest; Minv 884 /
+// 39, 2118 / 135, 2749 / 461).
+// Output by rows: 36 dofs 53 / 23 at one configuration, 1078 / 56 at 16,384, 4346 / 179 at
+// 65,536 (Minv 103 / 40, 2144 / 143, 8778 / 507; ABA derivatives 217 / 100, 4976 / 465,
+// 20586 / 1806).  Matrices of a few hundred bytes stay where they were, but for the
+// derivatives: one configuration is a few cache lines and the serial walk is short (6
+// dofs: equal up to 16,384, FP64 21 / 28 there; derivatives 64 / 58).
 // Batch-fastest output: as long as the lane-per-configuration kernel has less than about
 // one wave per SIMD to hide its serial walk (36 dofs CRBA 53 / 33 at 4,096, 53 / 46 at 8,192,
-// 53 / 67 at 16,384; FP64 58 / 50 at 4,096, 58 / 82 at 8,192; Minv 105 / 65 at 4,096,
-// 110 / 112 at 8,192).  FP64 Minv was one solve launch per column: 1627 / 352 at 16,384.
+// 53 / 67 at 16,384; FP64 58 / 50 at 4,096, 58 / 82 at 8,192; Minv 105 / 50 at 4,096, 110 /
+// 81 at 8,192, 124 / 143 at 16,384; 18 dofs 44 / 33, 46 / 37, 47 / 58; derivatives 36 dofs
+// 233 / 143 at 4,096, 239 / 264 at 8,192, FP64 766 / 485 at 8,192, 934 / 1028 at 16,384;
+// 18 dofs 79 / 68, 86 / 99, FP64 216 / 151, 242 / 246).  FP64 Minv was one solve launch per
+// column: 1627 / 287 at 16,384.
 bool treePays(TreeOp op, bool prebuilt, bool rows, int nv, int es, int64_t B) {
   if (!prebuilt) return true;
+  if (op == TreeOp::kDeriv) return rows || B * 4 <= (nv < 12 ? 2048 : 5120) * es;
   if (op == TreeOp::kMinv && es == 8) return true;
   if (rows) return nv * nv * es > 512;
   if (nv < 12) return false;
-  return op == TreeOp::kCrba ? B * es <= 32768 : B <= 6144;
+  return op == TreeOp::kCrba ? B * es <= 32768 : B <= 10240;
 }
 
 template<class S> bool treeCrba(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, View<S> M, int upper) {
@@ -193,6 +237,32 @@ template<class S> bool treeMinv(hipStream_t st, GM m, const S* mc, int64_t B, CV
   return true;
 }
 
+size_t treeDerivEntries(GM m) {
+  const TProg* g = prog(m);
+  return g ? (size_t)treeWsEntries(*g) : 0;
+}
+
+template<class S>
+bool treeAbaDeriv(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> Xq,
+                  View<S> Xv, View<S> Minv, S* ws) {
+  const TProg* g = prog(m);
+  if (!g || B <= 0) return false;
+  // segments per round of the solve: two workgroups per CU where that allows any
+  int R = 3;
+  while (R > 1 && treeSolveLds<S>(*g, R) > kLdsMax / 2) --R;
+  const size_t l1 = treeRneadLds<S>(*g), l2 = treeSolveLds<S>(*g, R);
+  if (!allow(&t_rnead<S>, l1) || !allow(&t_dsolve<S>, l2)) return false;
+  const unsigned grid = treeGrid(B);
+  const unsigned y = grid <= 168 ? 3 : 1;
+  hipLaunchKernelGGL((t_rnead<S>), dim3(grid), dim3(treeThreads(*g)), l1, st, *g, mc, B, q, v, a, ws);
+  hipLaunchKernelGGL((t_dsolve<S>), dim3(grid, y), dim3(treeThreads(*g)), l2, st, *g, B, (const S*)ws, Xq, Xv, Minv, R);
+  return true;
+}
+
+template bool treeAbaDeriv<float>(hipStream_t, GM, const float*, int64_t, CView<float>, CView<float>, CView<float>,
+                                  View<float>, View<float>, View<float>, float*);
+template bool treeAbaDeriv<double>(hipStream_t, GM, const double*, int64_t, CView<double>, CView<double>,
+                                   CView<double>, View<double>, View<double>, View<double>, double*);
 template bool treeCrba<float>(hipStream_t, GM, const float*, int64_t, CView<float>, View<float>, int);
 template bool treeCrba<double>(hipStream_t, GM, const double*, int64_t, CView<double>, View<double>, int);
 template bool treeMinv<float>(hipStream_t, GM, const float*, int64_t, CView<float>, View<float>);

@@ -28,12 +28,19 @@ TreeProgram* buildTreeProgram(int nj, const int* parents, const int* types, std:
 // Whether a call is faster on the tree-parallel kernels.  prebuilt: the tree has kernels of
 // its own; rows: the output keeps a configuration's elements together (rs == 1); es: bytes
 // of a scalar.
-enum class TreeOp { kCrba, kMinv };
+enum class TreeOp { kCrba, kMinv, kDeriv };
 bool treePays(TreeOp op, bool prebuilt, bool rows, int nv, int es, int64_t B);
 
 // Each returns false, having launched nothing, when the model has no tree program or its
 // state does not fit the LDS: the caller then runs the lane-per-configuration kernels.
 template<class S> bool treeCrba(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, View<S> M, int upper);
 template<class S> bool treeMinv(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, View<S> X);
+
+// RNEA derivatives at a and the ABA-derivative solve; ws: treeDerivEntries(m) scalars per
+// configuration, the batch rounded up to a multiple of 8.
+size_t treeDerivEntries(GM m);
+template<class S>
+bool treeAbaDeriv(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> Xq,
+                  View<S> Xv, View<S> Minv, S* ws);
 
 }  // namespace rbd

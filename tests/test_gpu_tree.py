@@ -13,7 +13,7 @@ import pytest
 
 import oracle
 import pinocchio_amd as pa
-from helpers import f32_round, inputs, rel_err_mats
+from helpers import f32_round, inputs, rel_err_cols, rel_err_mats
 from pinocchio_amd import models as M
 
 pytestmark = pytest.mark.gpu
@@ -83,3 +83,57 @@ def test_crba_padded_leading_dimension(ctx, pad):
             got, gap = o[:, :B].reshape(nv, nv, B).transpose(2, 1, 0), o[:, B:]
         assert rel_err_mats(got, ref).max() < 1e-5
         assert (gap == 7.0).all()
+
+
+@pytest.mark.parametrize("tree", range(len(TREES)))
+@pytest.mark.parametrize("dt,bar", [(torch.float32, 4e-4), (torch.float64, 1e-9)])
+def test_aba_derivatives(ctx, tree, dt, bar):
+    d = TREES[tree]()
+    for B in BATCHES:
+        q, v, _, tau = _inputs(d, B, dt)
+        ref = oracle.aba_derivatives(d, q, v, tau)
+        ddq = oracle.aba(d, q, v, tau)
+        for runtime in (False, True):
+            m = pa.Model(ctx, d, runtime_topology=runtime)
+            for layout in ("col", "batch"):
+                e = pa.Engine(m, layout)
+                out = e.aba_derivatives(*(_dev(x, layout, dt) for x in (q, v, tau)))
+                err = [rel_err_mats(e.mats_to_numpy(o, layout, d.nv), r).max() for o, r in zip(out[:3], ref[:3])]
+                a = out[3].double().cpu().numpy()
+                err.append(rel_err_cols(a.T if layout == "col" else a, ddq).max())
+                assert max(err) < bar, (d.name, B, layout, runtime, err)
+
+
+def test_aba_derivatives_in_chunks(ctx):
+    """A batch beyond one chunk of the packed workspace: bit-identical to its parts."""
+    d = M.humanoid36()
+    e = pa.Engine(pa.Model(ctx, d), "col")
+    B = 10_603
+    x = [_dev(y, "col", torch.float64) for y in (lambda t: (t[0], t[1], t[3]))(inputs(d, B))]
+    whole = e.aba_derivatives(*x)
+    for lo, hi in ((0, 300), (B - 331, B)):
+        part = e.aba_derivatives(*(y[lo:hi].contiguous() for y in x))
+        for a, b in zip(whole, part):
+            assert torch.equal(a[lo:hi], b)
+
+
+def test_aba_derivatives_captured_after_a_smaller_workspace(ctx):
+    """A capture for which only a smaller workspace was reserved takes the other route."""
+    d = M.quadruped18()
+    c = pa.Context(0)
+    e = pa.Engine(pa.Model(c, d), "batch")
+    big = [_dev(y, "batch", torch.float32) for y in (lambda t: (t[0], t[1], t[3]))(inputs(d, 20_000))]
+    small = [y[:, :3000].contiguous() for y in big]
+    e.aba_derivatives(*big)  # reserves for 20,000 configurations of the other route
+    out = [torch.empty((d.nv * d.nv, 3000), device="cuda") for _ in range(3)]
+    ddq = torch.empty((d.nv, 3000), device="cuda")
+    with c.capture() as cap:
+        e.aba_derivatives(*small, out=out, ddq_out=ddq, async_=True)
+    ref = e.aba_derivatives(*small)
+    for _ in range(3):
+        for o in (*out, ddq):
+            o.zero_()
+        torch.cuda.synchronize()
+        cap.graph.launch()
+        for a, b in zip((*out, ddq), ref):
+            assert ((a - b).abs().max() <= 2e-4 * b.abs().max()).item()
