@@ -20,6 +20,7 @@
 #pragma once
 
 #include "k_deriv.hpp"
+#include "k_dyn.hpp"
 
 namespace rbd {
 constexpr int kTreeT = 8;            // configurations per workgroup: 8 workers per wave
@@ -30,7 +31,9 @@ constexpr int kTreeMaxThreads = 1024;
 // are r + 1 .. r + sub[r] - 1, so entry (r, c) sits at rp[r] + c.  Offsets into tab:
 struct TProg {
   const int16_t* tab;
-  int nTab, nTabFactor;   // entries without and with the factorisation's lists
+  int nTabDyn, nTab, nTabFactor;  // entries RNEA and ABA need; and the matrices; and the factor
+  int oJLvl, oJList;      // joints by level of the tree
+  int oKidP, oKid;        // children of each joint
   int oJump;              // nlog x nj: the ancestor 2^k joints up (0: none)
   int oSubJ;              // per joint: joints of its subtree
   int oDofJ, oDl, oRp, oSub;  // per dof: joint, number of ancestor dofs, rp, subtree dofs
@@ -40,7 +43,7 @@ struct TProg {
   int oPairs;             // (r | c << 8) of the entries with r <= c; read from memory
   int oSeg, nseg;         // chain segments: first dof and length (up to four consecutive dofs)
   int oCommon;            // bytes, nv x nv: number of common strict ancestors of r and c
-  int nj, nq, nv, nlog, nnz;
+  int nj, nq, nv, nlev, nlog, nnz;
   uint32_t nvMagic;       // ceil(2^32 / nv): e / nv by multiplication for e < 2^16
 };
 enum : int { TJ_PARENT = 0, TJ_TYPE, TJ_IQ, TJ_IV, TJ_NV, TJ_REC };
@@ -806,6 +809,232 @@ __global__ __launch_bounds__(kTreeMaxThreads) void t_dsolve(TProg g, int64_t B, 
     __syncthreads();
   }
   // -- end
+}
+
+// ---------------------------------------------------------------------------------------
+// RNEA and ABA (rnea.hxx:17-161, aba.hxx:79-293; local frames and the re-associated bias of
+// k_dyn.hpp).  What does not depend on other joints (transforms, body inertias and forces)
+// is one phase over all joints; velocities and accelerations go down and forces and
+// articulated inertias up by levels of the tree, a parent adding what its children left in
+// their records.  Records: the joint transform (12), then
+//   RNEA: v, later the force; a, later the force moved to the parent;
+//   ABA: inertia (21) and bias force, later those moved to the parent; v, later the
+//   acceleration; the accumulated bias, later U / D; u / D - bias . U / D.
+// One workgroup's sweep is some 20 phases of short work for its few workers per level: two
+// waves and a small tile leave room for several workgroups per CU.
+// ---------------------------------------------------------------------------------------
+constexpr int kTreeDynC = 23;       // staged constants: placement, mass, lever, inertia
+constexpr int kTreeRneaJnt = 25, kTreeAbaJnt = 53;
+template<class S> size_t treeDynLds(const TProg& g, int rec) {
+  return (size_t)((g.nTabDyn + 7) & ~7) * 2 +
+         ((size_t)g.nj * (rec * kTreeT + kTreeDynC) + (size_t)(g.nq + 3 * g.nv) * kTreeT) * sizeof(S);
+}
+template<class S> __device__ __forceinline__ Mot<S> treeJointMot(int ty, const S* x) {  // S x of a joint's slice
+  if (ty == JT_FF)
+    return {{x[0], x[kTreeT], x[2 * kTreeT]}, {x[3 * kTreeT], x[4 * kTreeT], x[5 * kTreeT]}};
+  return axisMot(ty - JT_RX, x[0]);
+}
+template<class S> struct TreeDyn {  // LDS of a tile
+  int16_t* tb;
+  S *sj, *sc, *sq, *sv, *sx, *so;
+};
+// stages the tile's inputs and constants; so: nv rows of output
+template<class S>
+__device__ __forceinline__ TreeDyn<S> treeDynStage(const TProg& g, unsigned char* lds, int rec,
+                                                   const S* __restrict__ mc, CView<S> gq, CView<S> gv, CView<S> gx,
+                                                   int64_t b0, int nb) {
+  TreeDyn<S> t;
+  t.tb = reinterpret_cast<int16_t*>(lds);
+  t.sj = reinterpret_cast<S*>(t.tb + ((g.nTabDyn + 7) & ~7));
+  t.sc = t.sj + g.nj * rec * kTreeT;
+  t.sq = t.sc + g.nj * kTreeDynC;
+  t.sv = t.sq + g.nq * kTreeT;
+  t.sx = t.sv + g.nv * kTreeT;
+  t.so = t.sx + g.nv * kTreeT;
+  treeStageTab(g, t.tb, g.nTabDyn);
+  treeStageConsts<S, MC_R, 12, kTreeDynC, 0>(mc, g.nj, t.sc);
+  treeStageConsts<S, MC_M, 10, kTreeDynC, 12>(mc, g.nj, t.sc);
+  treeStage(t.sq, gq, g.nq, b0, nb);
+  treeStage(t.sv, gv, g.nv, b0, nb);
+  treeStage(t.sx, gx, g.nv, b0, nb);
+  __syncthreads();
+  return t;
+}
+template<class S>
+__device__ __forceinline__ void treeDynOut(const S* so, View<S> g, int R, int64_t b0, int nb) {
+  __syncthreads();
+  if (g.rs == 1) {
+    for (int e = threadIdx.x; e < R * nb; e += blockDim.x) {
+      const int b = e / R, k = e - b * R;
+      g.p[(b0 + b) * g.bs + k] = so[k * kTreeT + b];
+    }
+  } else {
+    for (int e = threadIdx.x; e < R * kTreeT; e += blockDim.x) {
+      const int k = e / kTreeT, b = e % kTreeT;
+      if (b < nb) g.p[k * g.rs + (b0 + b) * g.bs] = so[e];
+    }
+  }
+}
+template<class S>
+__global__ __launch_bounds__(kTreeMaxThreads) void t_rnea(TProg g, const S* __restrict__ mc, int64_t B, CView<S> gq,
+                                                          CView<S> gv, CView<S> ga, View<S> gtau) {
+  extern __shared__ __align__(16) unsigned char t_lds[];
+  const int64_t b0 = treeTile() * kTreeT;
+  if (b0 >= B) return;
+  const int nb = (int)(B - b0 < kTreeT ? B - b0 : kTreeT);
+  const TreeDyn<S> t = treeDynStage(g, t_lds, kTreeRneaJnt, mc, gq, gv, ga, b0, nb);
+  const int16_t* tb = t.tb;
+  const int b = treeB(), w = treeW(), NW = treeNW();
+  const S* __restrict__ arm = mc + g.nj * MC_REC;
+  const Mot<S> a0 = mcGravityNeg(arm, g.nv);
+  auto jnt = [&](int j) { return TRec<S>{t.sj + j * kTreeRneaJnt * kTreeT + b}; };
+  for (int j = 1 + w; j < g.nj; j += NW)
+    jnt(j).put(0, treeJointX(t.sc + j * kTreeDynC, tb[j * TJ_REC + TJ_TYPE], t.sq + b, tb[j * TJ_REC + TJ_IQ]));
+  for (int l = 0; l < g.nlev; ++l) {
+    __syncthreads();
+    for (int e = tb[g.oJLvl + l] + w, e1 = tb[g.oJLvl + l + 1]; e < e1; e += NW) {
+      const int j = tb[g.oJList + e], p = tb[j * TJ_REC + TJ_PARENT], ty = tb[j * TJ_REC + TJ_TYPE];
+      const int iv = tb[j * TJ_REC + TJ_IV];
+      const Xform<S> X = jnt(j).template get<Xform<S>>(0);
+      const Mot<S> vJ = treeJointMot(ty, t.sv + iv * kTreeT + b);
+      Mot<S> v = vJ, a = treeJointMot(ty, t.sx + iv * kTreeT + b);
+      if (p > 0) {
+        v = v + actInv(X, jnt(p).template get<Mot<S>>(12));
+        a = a + actInv(X, jnt(p).template get<Mot<S>>(18));
+      } else {
+        a = a + actInv(X, a0);
+      }
+      jnt(j).put(12, v);
+      jnt(j).put(18, a + crossMM(v, vJ));
+    }
+  }
+  __syncthreads();
+  for (int j = 1 + w; j < g.nj; j += NW) {
+    const Body<S> Y = ldsConst<Body<S>>(t.sc + j * kTreeDynC + 12);
+    const Mot<S> v = jnt(j).template get<Mot<S>>(12);
+    jnt(j).put(12, inertiaMul(Y, jnt(j).template get<Mot<S>>(18)) + crossMF(v, inertiaMul(Y, v)));
+  }
+  for (int l = g.nlev - 1; l >= 0; --l) {
+    __syncthreads();
+    for (int e = tb[g.oJLvl + l] + w, e1 = tb[g.oJLvl + l + 1]; e < e1; e += NW) {
+      const int j = tb[g.oJList + e], ty = tb[j * TJ_REC + TJ_TYPE], iv = tb[j * TJ_REC + TJ_IV];
+      Frc<S> f = jnt(j).template get<Frc<S>>(12);
+      for (int k = tb[g.oKidP + j], k1 = tb[g.oKidP + j + 1]; k < k1; ++k)
+        f = f + jnt(tb[g.oKid + k]).template get<Frc<S>>(18);
+      if (ty == JT_FF) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k)
+          t.so[(iv + k) * kTreeT + b] = comp(f, k) + arm[iv + k] * t.sx[(iv + k) * kTreeT + b];
+      } else {
+        t.so[iv * kTreeT + b] = comp(f.a, ty - JT_RX) + arm[iv] * t.sx[iv * kTreeT + b];
+      }
+      if (l > 0) jnt(j).put(18, act(jnt(j).template get<Xform<S>>(0), f));
+    }
+  }
+  treeDynOut(t.so, gtau, g.nv, b0, nb);
+}
+
+template<class S>
+__global__ __launch_bounds__(kTreeMaxThreads) void t_aba(TProg g, const S* __restrict__ mc, int64_t B, CView<S> gq,
+                                                         CView<S> gv, CView<S> gt, View<S> gddq) {
+  extern __shared__ __align__(16) unsigned char t_lds[];
+  const int64_t b0 = treeTile() * kTreeT;
+  if (b0 >= B) return;
+  const int nb = (int)(B - b0 < kTreeT ? B - b0 : kTreeT);
+  const TreeDyn<S> t = treeDynStage(g, t_lds, kTreeAbaJnt, mc, gq, gv, gt, b0, nb);
+  const int16_t* tb = t.tb;
+  const int b = treeB(), w = treeW(), NW = treeNW();
+  const S* __restrict__ arm = mc + g.nj * MC_REC;
+  const Mot<S> a0 = mcGravityNeg(arm, g.nv);
+  constexpr int kI = 12, kP = 33, kV = 39, kC = 45, kS = 51;  // inertia, force, v, bias, scalar
+  auto jnt = [&](int j) { return TRec<S>{t.sj + j * kTreeAbaJnt * kTreeT + b}; };
+  for (int j = 1 + w; j < g.nj; j += NW)
+    jnt(j).put(0, treeJointX(t.sc + j * kTreeDynC, tb[j * TJ_REC + TJ_TYPE], t.sq + b, tb[j * TJ_REC + TJ_IQ]));
+  for (int l = 0; l < g.nlev; ++l) {
+    __syncthreads();
+    for (int e = tb[g.oJLvl + l] + w, e1 = tb[g.oJLvl + l + 1]; e < e1; e += NW) {
+      const int j = tb[g.oJList + e], p = tb[j * TJ_REC + TJ_PARENT], ty = tb[j * TJ_REC + TJ_TYPE];
+      const Xform<S> X = jnt(j).template get<Xform<S>>(0);
+      const Mot<S> vJ = treeJointMot(ty, t.sv + tb[j * TJ_REC + TJ_IV] * kTreeT + b);
+      Mot<S> v = vJ;
+      if (p > 0) v = v + actInv(X, jnt(p).template get<Mot<S>>(kV));
+      Mot<S> c = crossMM(v, vJ);
+      if (p > 0) c = c + actInv(X, jnt(p).template get<Mot<S>>(kC));
+      jnt(j).put(kV, v);
+      jnt(j).put(kC, c);
+    }
+  }
+  __syncthreads();
+  for (int j = 1 + w; j < g.nj; j += NW) {
+    const Body<S> Y = ldsConst<Body<S>>(t.sc + j * kTreeDynC + 12);
+    const Mot<S> v = jnt(j).template get<Mot<S>>(kV);
+    jnt(j).put(kP, crossMF(v, inertiaMul(Y, v)));
+    jnt(j).put(kI, bodyMatrix(Y));
+  }
+  for (int l = g.nlev - 1; l >= 0; --l) {
+    __syncthreads();
+    for (int e = tb[g.oJLvl + l] + w, e1 = tb[g.oJLvl + l + 1]; e < e1; e += NW) {
+      const int j = tb[g.oJList + e], p = tb[j * TJ_REC + TJ_PARENT], ty = tb[j * TJ_REC + TJ_TYPE];
+      const int iv = tb[j * TJ_REC + TJ_IV];
+      Sym6<S> Ia = jnt(j).template get<Sym6<S>>(kI);
+      Frc<S> pA = jnt(j).template get<Frc<S>>(kP);
+      for (int k = tb[g.oKidP + j], k1 = tb[g.oKidP + j + 1]; k < k1; ++k) {
+        const int c = tb[g.oKid + k];
+        symAdd(Ia, jnt(c).template get<Sym6<S>>(kI));
+        pA = pA + jnt(c).template get<Frc<S>>(kP);
+      }
+      const Xform<S> X = jnt(j).template get<Xform<S>>(0);
+      if (ty == JT_FF) {
+        // root free flyer: D = Ia + armature (6x6, FP64 LLT), qdd = D^-1 (tau - pA - Ia a')
+        const Mot<S> ap = actInv(X, a0);
+        const Frc<S> Iap = symMul6(Ia, ap);
+        double A[21], x[6];
+#pragma unroll
+        for (int r = 0; r < 6; ++r) {
+#pragma unroll
+          for (int c = 0; c <= r; ++c) A[lowIdx(r, c)] = double(sget(Ia, r, c));
+          A[lowIdx(r, r)] += double(arm[iv + r]);
+          x[r] = double(t.sx[(iv + r) * kTreeT + b]) - double(comp(pA, r)) - double(comp(Iap, r));
+        }
+        spdSolve6(A, x);
+#pragma unroll
+        for (int r = 0; r < 6; ++r) t.so[(iv + r) * kTreeT + b] = S(x[r]);
+        jnt(j).put(kV, Mot<S>{{ap.l.x + S(x[0]), ap.l.y + S(x[1]), ap.l.z + S(x[2])},
+                              {ap.a.x + S(x[3]), ap.a.y + S(x[4]), ap.a.z + S(x[5])}});
+      } else {
+        const int ax = ty - JT_RX;
+        const Frc<S> c3 = symCol(Ia, 3), c4 = symCol(Ia, 4), c5 = symCol(Ia, 5);
+        auto sel = [&](S x, S y, S z) { return ax == 0 ? x : (ax == 1 ? y : z); };
+        const Frc<S> U = {{sel(c3.l.x, c4.l.x, c5.l.x), sel(c3.l.y, c4.l.y, c5.l.y), sel(c3.l.z, c4.l.z, c5.l.z)},
+                          {sel(c3.a.x, c4.a.x, c5.a.x), sel(c3.a.y, c4.a.y, c5.a.y), sel(c3.a.z, c4.a.z, c5.a.z)}};
+        const S Dinv = S(1) / (comp(U.a, ax) + arm[iv]);
+        const S u = t.sx[iv * kTreeT + b] - comp(pA.a, ax);
+        const Frc<S> dd = scale(Dinv, U);
+        const Mot<S> c = jnt(j).template get<Mot<S>>(kC);
+        t.sj[(j * kTreeAbaJnt + kS) * kTreeT + b] = Dinv * u - dot(c, dd);
+        jnt(j).put(kC, dd);
+        if (p > 0) {
+          symRank1Sub(Ia, U, Dinv);
+          const Mot<S> ci = crossMM(jnt(j).template get<Mot<S>>(kV), axisMot(ax, t.sv[iv * kTreeT + b]));
+          const Frc<S> pa = pA + symMul6(Ia, ci) + scale(Dinv * u, U);
+          jnt(j).put(kI, transportUp(X, Ia));
+          jnt(j).put(kP, act(X, pa));
+        }
+      }
+    }
+  }
+  for (int l = 0; l < g.nlev; ++l) {
+    __syncthreads();
+    for (int e = tb[g.oJLvl + l] + w, e1 = tb[g.oJLvl + l + 1]; e < e1; e += NW) {
+      const int j = tb[g.oJList + e], p = tb[j * TJ_REC + TJ_PARENT], ty = tb[j * TJ_REC + TJ_TYPE];
+      if (ty == JT_FF) continue;
+      const Mot<S> x = actInv(jnt(j).template get<Xform<S>>(0), p > 0 ? jnt(p).template get<Mot<S>>(kV) : a0);
+      const S qdd = t.sj[(j * kTreeAbaJnt + kS) * kTreeT + b] - dot(x, jnt(j).template get<Frc<S>>(kC));
+      t.so[tb[j * TJ_REC + TJ_IV] * kTreeT + b] = qdd;
+      jnt(j).put(kV, x + axisMot(ty - JT_RX, qdd));
+    }
+  }
+  treeDynOut(t.so, gddq, g.nv, b0, nb);
 }
 
 }  // namespace rbd

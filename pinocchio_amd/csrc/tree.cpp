@@ -61,6 +61,22 @@ TreeProgram* buildTreeProgram(int nj, const int* parents, const int* types, std:
     return o;
   };
   for (int j = 0; j < nj; ++j) flat({parents[j], types[j], iq[j], iv[j], nvj[j]});
+  // a list grouped by key 0 .. n - 1 of the joints: group starts, then the members
+  auto grouped = [&](int n, auto key, int& oPtr, int& oList) {
+    std::vector<int> ptr, list;
+    for (int k = 0; k < n; ++k) {
+      ptr.push_back((int)list.size());
+      for (int j = 1; j < nj; ++j)
+        if (key(j) == k) list.push_back(j);
+    }
+    ptr.push_back((int)list.size());
+    oPtr = flat(ptr);
+    oList = flat(list);
+  };
+  g.nlev = maxDepth;
+  grouped(maxDepth, [&](int j) { return depth[j] - 1; }, g.oJLvl, g.oJList);
+  grouped(nj, [&](int j) { return parents[j]; }, g.oKidP, g.oKid);
+  g.nTabDyn = (int)tab.size();
   std::vector<int> up(parents, parents + nj);
   g.oJump = (int)tab.size();
   for (; (1 << g.nlog) < maxDepth; ++g.nlog) {
@@ -219,6 +235,14 @@ bool treePays(TreeOp op, bool prebuilt, bool rows, int nv, int es, int64_t B) {
   return op == TreeOp::kCrba ? B * es <= 32768 : B <= 10240;
 }
 
+// The tree-parallel sweeps take a few phases per level with most lanes idle, so they win
+// until the lane-per-configuration ones fill the chip: that is later for a shallow tree.
+// us per call, run-time topology / tree-parallel: RNEA 10 levels (36 dofs) 72 / 33 at one
+// configuration, 80 / 57 at 16,384, 172 / 179 at 65,536; 40 levels (a chain) 110 / 75 at
+// 4,096, 112 / 131 at 8,192.  ABA 10 levels 224 / 45, 309 / 139, 489 / 510; 40 levels 475 /
+// 453 at 16,384; 4 levels (18 dofs) 63 / 29 at one, 118 / 118 at 65,536, FP64 243 / 286.
+bool treeDynPays(bool aba, int nlev, int es, int64_t B) { return B * es * nlev <= (aba ? 1400000 : 655360); }
+
 template<class S> bool treeCrba(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, View<S> M, int upper) {
   const TProg* g = prog(m);
   if (!g || B <= 0) return false;
@@ -236,6 +260,35 @@ template<class S> bool treeMinv(hipStream_t st, GM m, const S* mc, int64_t B, CV
   hipLaunchKernelGGL((t_minv<S>), dim3(treeGrid(B)), dim3(treeThreads(*g)), lds, st, *g, mc, B, q, X);
   return true;
 }
+
+// RNEA and ABA: a level has few joints; 16 workers
+constexpr unsigned kTreeDynThreads = 128;
+template<class S>
+bool treeRnea(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> tau) {
+  const TProg* g = prog(m);
+  if (!g || B <= 0) return false;
+  const size_t lds = treeDynLds<S>(*g, kTreeRneaJnt);
+  if (!allow(&t_rnea<S>, lds)) return false;
+  hipLaunchKernelGGL((t_rnea<S>), dim3(treeGrid(B)), dim3(kTreeDynThreads), lds, st, *g, mc, B, q, v, a, tau);
+  return true;
+}
+template<class S>
+bool treeAba(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> tau, View<S> ddq) {
+  const TProg* g = prog(m);
+  if (!g || B <= 0) return false;
+  const size_t lds = treeDynLds<S>(*g, kTreeAbaJnt);
+  if (!allow(&t_aba<S>, lds)) return false;
+  hipLaunchKernelGGL((t_aba<S>), dim3(treeGrid(B)), dim3(kTreeDynThreads), lds, st, *g, mc, B, q, v, tau, ddq);
+  return true;
+}
+template bool treeRnea<float>(hipStream_t, GM, const float*, int64_t, CView<float>, CView<float>, CView<float>,
+                              View<float>);
+template bool treeRnea<double>(hipStream_t, GM, const double*, int64_t, CView<double>, CView<double>, CView<double>,
+                               View<double>);
+template bool treeAba<float>(hipStream_t, GM, const float*, int64_t, CView<float>, CView<float>, CView<float>,
+                             View<float>);
+template bool treeAba<double>(hipStream_t, GM, const double*, int64_t, CView<double>, CView<double>, CView<double>,
+                              View<double>);
 
 size_t treeDerivEntries(GM m) {
   const TProg* g = prog(m);

@@ -30,11 +30,17 @@ TreeProgram* buildTreeProgram(int nj, const int* parents, const int* types, std:
 // of a scalar.
 enum class TreeOp { kCrba, kMinv, kDeriv };
 bool treePays(TreeOp op, bool prebuilt, bool rows, int nv, int es, int64_t B);
+// RNEA and ABA of a tree without kernels of its own; nlev: levels of the tree
+bool treeDynPays(bool aba, int nlev, int es, int64_t B);
 
 // Each returns false, having launched nothing, when the model has no tree program or its
 // state does not fit the LDS: the caller then runs the lane-per-configuration kernels.
 template<class S> bool treeCrba(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, View<S> M, int upper);
 template<class S> bool treeMinv(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, View<S> X);
+template<class S>
+bool treeRnea(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> tau);
+template<class S>
+bool treeAba(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> tau, View<S> ddq);
 
 // RNEA derivatives at a and the ABA-derivative solve; ws: treeDerivEntries(m) scalars per
 // configuration, the batch rounded up to a multiple of 8.

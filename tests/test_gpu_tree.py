@@ -61,6 +61,25 @@ def test_crba_and_minverse(ctx, tree, dt, bar, bar_inv):
                 assert rel_err_mats(num(e.compute_minverse(x)), inv).max() < bar_inv, (d.name, B, layout)
 
 
+@pytest.mark.parametrize("tree", range(len(TREES)))
+@pytest.mark.parametrize("dt,bar_rnea,bar_aba", [(torch.float32, 1e-5, 1e-4), (torch.float64, 1e-12, 1e-10)])
+def test_rnea_and_aba(ctx, tree, dt, bar_rnea, bar_aba):
+    d = TREES[tree]()
+    m = pa.Model(ctx, d, runtime_topology=True)
+    for B in BATCHES:
+        q, v, a, tau = _inputs(d, B, dt)
+        refs = oracle.rnea(d, q, v, a), oracle.aba(d, q, v, tau)
+        for layout in ("col", "batch"):
+            e = pa.Engine(m, layout)
+            Q, V, A, T = (_dev(x, layout, dt) for x in (q, v, a, tau))
+            for out, ref, bar in ((e.rnea(Q, V, A), refs[0], bar_rnea), (e.aba(Q, V, T), refs[1], bar_aba)):
+                x = out.double().cpu().numpy()
+                assert rel_err_cols(x.T if layout == "col" else x, ref).max() < bar, (d.name, B, layout)
+        e = pa.Engine(m, "col")  # inputs that are zero for every configuration
+        g = e.generalized_gravity(_dev(q, "col", dt)).double().cpu().numpy().T
+        assert rel_err_cols(g, oracle.rnea(d, q, 0 * v, 0 * a)).max() < 2 * bar_rnea, (d.name, B)
+
+
 @pytest.mark.parametrize("pad", [1, 3, 4])
 def test_crba_padded_leading_dimension(ctx, pad):
     """Rows that are not 16-byte aligned, and gaps that stay as the caller had them."""
