@@ -143,7 +143,10 @@ void launchAbaDSolve(hipStream_t st, GM, int64_t B, CView<S> U, CView<S> D, View
 template<class TP, class S>
 void launchKin(hipStream_t st, GM, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> oM, View<S> vo,
                View<S> ao, View<S> J) {
-  hipLaunchKernelGGL((k_kin<TP, S>), dim3(gridFor(B)), dim3(kTile), 0, st, mc, B, q, v, a, oM, vo, ao, J);
+  if (kinRows(oM, vo, ao, J))
+    hipLaunchKernelGGL((k_kin<TP, S, true>), dim3(gridFor(B)), dim3(kTile), 0, st, mc, B, q, v, a, oM, vo, ao, J);
+  else
+    hipLaunchKernelGGL((k_kin<TP, S, false>), dim3(gridFor(B)), dim3(kTile), 0, st, mc, B, q, v, a, oM, vo, ao, J);
 }
 
 template<class TP, class S>

@@ -32,6 +32,7 @@
 
 #include "k_deriv.hpp"
 #include "k_dyn.hpp"
+#include "k_kin.hpp"
 
 namespace rbd {
 
@@ -651,10 +652,10 @@ __global__ __launch_bounds__(64 * kGSolveWaves) void g_abad_solve(GProg g, int64
 // Forward kinematics and WORLD joint Jacobians (kinematics.hxx:121-145, 209-238;
 // jacobian.hxx:23-62); outputs as k_kin.hpp, any may be absent.
 // ---------------------------------------------------------------------------------------
-template<class S, bool kLds>
-__global__ __launch_bounds__(64) void g_kin(GProg g, const S* __restrict__ mc, int64_t B, CView<S> gq, CView<S> gv,
-                                            CView<S> ga, View<S> gM, View<S> gV, View<S> gA, View<S> gJ,
-                                            S* __restrict__ ws) {
+template<class S, bool kLds, bool kRows>
+__device__ __forceinline__ void gKinTiles(GProg g, const S* __restrict__ mc, int64_t B, CView<S> gq, CView<S> gv,
+                                          CView<S> ga, View<S> gM, View<S> gV, View<S> gA, View<S> gJ,
+                                          S* __restrict__ ws) {
   const int L = laneId();
   const Lane<S> m = laneMem<S, kLds>(ws, (int64_t)g.nlev * kGKinLvl * kTile);
   const bool wantV = gV.p != nullptr, wantA = gA.p != nullptr;
@@ -663,8 +664,15 @@ __global__ __launch_bounds__(64) void g_kin(GProg g, const S* __restrict__ mc, i
     const int nb = (int)(B - b0 < kTile ? B - b0 : kTile);
     const bool live = L < nb;
     const int64_t b = b0 + (live ? L : nb - 1);
-    auto put = [&](View<S> o, int row, S x) {
-      if (live) stOut(&o.p[(int64_t)row * o.rs + b * o.bs], x);
+    auto put = [&](auto Nc, View<S> o, int row, const S* x) {
+      constexpr int N = Nc;
+      if (!live) return;
+      if constexpr (kRows) {
+        putRun<N>(o.p + b * o.bs + row, x);
+      } else {
+#pragma unroll
+        for (int k = 0; k < N; ++k) stOut(&o.p[(int64_t)(row + k) * o.rs + b * o.bs], x[k]);
+      }
     };
     for (int e = 0; e < g.nev; ++e) {
       const int ev = g.ev[e];
@@ -679,8 +687,7 @@ __global__ __launch_bounds__(64) void g_kin(GProg g, const S* __restrict__ mc, i
       if (gM.p) {
         const R3<S>& R = oM.R;
         const S r12[12] = {R.m00, R.m01, R.m02, R.m10, R.m11, R.m12, R.m20, R.m21, R.m22, oM.p.x, oM.p.y, oM.p.z};
-#pragma unroll
-        for (int k = 0; k < 12; ++k) put(gM, (i - 1) * 12 + k, r12[k]);
+        put(IC<12>{}, gM, (i - 1) * 12, r12);
       }
       if (wantV) {
         const Mot<S> vJ = gJointMot(ty, gv, iv, b);
@@ -688,27 +695,38 @@ __global__ __launch_bounds__(64) void g_kin(GProg g, const S* __restrict__ mc, i
         if (p > 0) vi = vi + actInv(X, m.template get<Mot<S>>(sp + 12));
         m.put(s0 + 12, vi);
         const S o[6] = {vi.l.x, vi.l.y, vi.l.z, vi.a.x, vi.a.y, vi.a.z};
-#pragma unroll
-        for (int k = 0; k < 6; ++k) put(gV, (i - 1) * 6 + k, o[k]);
+        put(IC<6>{}, gV, (i - 1) * 6, o);
         if (wantA) {
           Mot<S> ai = crossMM(vi, vJ) + gJointMot(ty, ga, iv, b);
           if (p > 0) ai = ai + actInv(X, m.template get<Mot<S>>(sp + 18));
           m.put(s0 + 18, ai);
           const S oa[6] = {ai.l.x, ai.l.y, ai.l.z, ai.a.x, ai.a.y, ai.a.z};
-#pragma unroll
-          for (int k = 0; k < 6; ++k) put(gA, (i - 1) * 6 + k, oa[k]);
+          put(IC<6>{}, gA, (i - 1) * 6, oa);
         }
       }
       if (gJ.p) {
         for (int k = 0; k < nvi; ++k) {
           const Mot<S> c = gWorldAxis(ty, oM, k);
           const S o[6] = {c.l.x, c.l.y, c.l.z, c.a.x, c.a.y, c.a.z};
-#pragma unroll
-          for (int r = 0; r < 6; ++r) put(gJ, (iv + k) * 6 + r, o[r]);
+          put(IC<6>{}, gJ, (iv + k) * 6, o);
         }
       }
     }
   }
+}
+
+template<class S, bool kLds>
+__global__ __launch_bounds__(64) void g_kin(GProg g, const S* __restrict__ mc, int64_t B, CView<S> gq, CView<S> gv,
+                                            CView<S> ga, View<S> gM, View<S> gV, View<S> gA, View<S> gJ,
+                                            S* __restrict__ ws) {
+  gKinTiles<S, kLds, false>(g, mc, B, gq, gv, ga, gM, gV, gA, gJ, ws);
+}
+// outputs by rows (kinRows)
+template<class S, bool kLds>
+__global__ __launch_bounds__(64) void g_kin_rows(GProg g, const S* __restrict__ mc, int64_t B, CView<S> gq, CView<S> gv,
+                                                 CView<S> ga, View<S> gM, View<S> gV, View<S> gA, View<S> gJ,
+                                                 S* __restrict__ ws) {
+  gKinTiles<S, kLds, true>(g, mc, B, gq, gv, ga, gM, gV, gA, gJ, ws);
 }
 
 }  // namespace rbd

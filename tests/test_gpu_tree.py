@@ -1,4 +1,4 @@
-"""Tree-parallel kernels against the FP64 oracle at the sizes where their tiles of eight
+"""Tree-parallel kernels and vector stores of row outputs against the FP64 oracle at the sizes where their tiles of eight
 configurations, levels and rounds can go wrong, on every route of the dispatch (prebuilt
 and run-time topologies, both layouts and precisions, padded leading dimensions).
 
@@ -156,3 +156,34 @@ def test_aba_derivatives_captured_after_a_smaller_workspace(ctx):
         cap.graph.launch()
         for a, b in zip((*out, ddq), ref):
             assert ((a - b).abs().max() <= 2e-4 * b.abs().max()).item()
+
+
+@pytest.mark.parametrize("dt,bar", [(torch.float32, 2e-6), (torch.float64, 1e-13)])
+@pytest.mark.parametrize("pad", [0, 1, 2, 4])
+def test_kinematics_rows(ctx, dt, bar, pad):
+    """Row outputs whose runs are and are not aligned to the vector stores, with gaps that stay
+    as the caller had them; against the oracle (FP32: rounding of at most 30 composed
+    placements in one coordinate of the largest)."""
+    for d, runtime in ((M.arm7(), False), (M.humanoid36(), False), (M.humanoid36(), True), (M.random_tree(12, 5), False)):
+        m = pa.Model(ctx, d, runtime_topology=runtime)
+        nj, nv, B = d.njoints - 1, d.nv, 131
+        q, v, a, _ = _inputs(d, B, dt)
+        Q, V, A = (_dev(x, "col", dt) for x in (q, v, a))
+        rows = {"M": 12 * nj, "v": 6 * nj, "a": 6 * nj, "J": 6 * nv}
+        out = {k: torch.full((B, n + pad), 7.0, dtype=dt, device="cuda") for k, n in rows.items()}
+        code = pa.RBD_F32 if dt == torch.float32 else pa.RBD_F64
+        p, i = pa._ptr, pa._i64
+        pa._check(pa.lib().rbd_forward_kinematics(
+            ctx.handle, m.handle, i(B), code, p(Q), i(d.nq), p(V), i(nv), p(A), i(nv), p(out["M"]),
+            i(out["M"].stride(0)), p(out["v"]), p(out["a"]), i(out["v"].stride(0)), ctypes.c_uint32(0)))
+        pa._check(pa.lib().rbd_joint_jacobians(ctx.handle, m.handle, i(B), code, p(Q), i(d.nq), p(out["J"]),
+                                               i(out["J"].stride(0)), ctypes.c_uint32(0)))
+        oM, ov, oa = oracle.forward_kinematics(d, q, v, a)
+        ref = {"M": oM[:, 1:].reshape(B, -1) if oM.shape[1] == nj + 1 else oM.reshape(B, -1),
+               "v": ov[:, 1:].reshape(B, -1) if ov.shape[1] == nj + 1 else ov.reshape(B, -1),
+               "a": oa[:, 1:].reshape(B, -1) if oa.shape[1] == nj + 1 else oa.reshape(B, -1),
+               "J": oracle.joint_jacobians(d, q).transpose(0, 2, 1).reshape(B, -1)}
+        for k, n in rows.items():
+            x = out[k].double().cpu().numpy()
+            assert rel_err_cols(x[:, :n].T, ref[k].T).max() < bar, (d.name, k, pad)
+            assert (x[:, n:] == 7.0).all()
