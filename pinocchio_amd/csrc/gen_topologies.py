@@ -36,10 +36,14 @@ _RNEAD = ("const float*, int64_t, CView<float>, CView<float>, CView<float>, View
           "View<float>, int")
 WAVE_KERNELS = {
     "dyn": [("k_aba_waves", "float", _VEC3.format(s="float"), (2, 4)),
-            ("k_aba_waves", "double", _VEC3.format(s="double"), (4,))],
+            ("k_aba_waves", "double", _VEC3.format(s="double"), (4,)),
+            ("k_rnea_waves", "float", _VEC3.format(s="float"), (4,)),
+            ("k_rnea_waves", "double", _VEC3.format(s="double"), (4,))],
     "rnead": [("k_rnead", "float", _RNEAD, (4,))],
 }
+WAVE_TAG = {"k_rnea_waves": "rnea_"}  # units of a family's second multi-wave kernel
 WAVE_COND = {"k_aba_waves": "abaSplitPaysFor<Topo_{name}, {sc}, {g}>()",
+             "k_rnea_waves": "rneaSplitPaysFor<Topo_{name}, {sc}, {g}>()",
              "k_rnead": "rneadSplitPays<Topo_{name}, {g}>()"}
 
 DYN = ["dyn", "kin"]
@@ -166,7 +170,7 @@ def main(out_dir=None, robots=""):
             for k, sc, sig, gs in WAVE_KERNELS.get(fam, []):
                 for g in gs:
                     cond = WAVE_COND[k].format(name=name, g=g, sc=sc)
-                    tag = f"w{g}" + ("" if sc == "float" else "d")
+                    tag = f"{WAVE_TAG.get(k, '')}w{g}" + ("" if sc == "float" else "d")
                     _write(os.path.join(out_dir, f"inst_{name}_{fam}_{tag}.hip"),
                            "// generated by gen_topologies.py -- do not edit\n"
                            "#include \"../instantiate.hpp\"\nnamespace rbd {\n"

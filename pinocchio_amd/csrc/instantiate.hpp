@@ -13,10 +13,6 @@ namespace rbd {
 
 inline unsigned gridFor(int64_t B) { return (unsigned)((B + kTile - 1) / kTile); }
 
-template<class TP, class S>
-void launchRnea(hipStream_t st, GM, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> out) {
-  hipLaunchKernelGGL((k_rnea<TP, S>), dim3(gridFor(B)), dim3(kTile), 0, st, mc, B, q, v, a, out);
-}
 // Below about four tiles per CU the sweeps are latency-bound with one wave per tile.
 inline int wavesForBatch(int64_t B) {
   const int64_t tiles = (B + kTile - 1) / kTile;
@@ -33,6 +29,28 @@ template<class TP, int G> constexpr bool abaSplitPays() {
 // ... and its LDS (sized for 4-byte scalars) fits at the scalar's width
 template<class TP, class S, int G> constexpr bool abaSplitPaysFor() {
   return abaSplitPays<TP, G>() && abaWavesLdsBytes<TP, G>() / 4 * (int)sizeof(S) <= 160 * 1024;
+}
+template<class TP, class S, int G> constexpr bool rneaSplitPaysFor() {
+  constexpr WaveSplit<TP, G> WS{};
+  int trunk = 0, busiest = 0;
+  for (int j = 1; j < TP::NJ; ++j) trunk += WS.owner[j] < 0 ? 1 : 0;
+  for (int k = 0; k < G; ++k) busiest = WS.load[k] > busiest ? WS.load[k] : busiest;
+  return 5 * (trunk + busiest) <= 3 * (TP::NJ - 1) && rneaWavesLdsBytes<TP, G>() / 4 * (int)sizeof(S) <= 160 * 1024;
+}
+// Four waves per tile wherever the tree splits (us per call, one wave / four: 18 dofs 30 / 22
+// at 512 rows, 53 / 49 at 200,000; 36 dofs 46 / 29, 126 / 99; FP64 295 / 208), but for FP32
+// tiles of which fewer than four fit a CU and more than fit the chip: the 60-dof tree 67 / 52
+// at 4,096 and 68 / 54 at 16,384, 132 / 160 at 65,536.
+template<class TP, class S>
+void launchRnea(hipStream_t st, GM, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> out) {
+  if constexpr (rneaSplitPaysFor<TP, S, 4>()) {
+    constexpr int perCu = 160 * 1024 / (rneaWavesLdsBytes<TP, 4>() / 4 * (int)sizeof(S));
+    if (sizeof(S) == 8 || perCu >= 4 || B <= (int64_t)perCu * 256 * kTile) {
+      hipLaunchKernelGGL((k_rnea_waves<TP, S, 4>), dim3(gridFor(B)), dim3(kTile * 4), 0, st, mc, B, q, v, a, out);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_rnea<TP, S>), dim3(gridFor(B)), dim3(kTile), 0, st, mc, B, q, v, a, out);
 }
 // RNEA derivatives: the same test, with the LDS of the staged inputs and the 43-float
 // subtree slots

@@ -40,32 +40,46 @@ template<class TP> constexpr int dynLdsRows() { return TP::T.nq + 2 * TP::T.nv; 
 // One 64-configuration tile starting at b0; `lds` holds dynLdsRows<TP>() * kPitch scalars.
 // (kU: loads in flight per lane while staging; the fused mixed-batch kernel, already at
 // the register limit, stages one row at a time)
-template<class TP, class S, int kU = kStageU>
+// G > 1: G waves share the tile and split the tree by subtrees (WaveSplit, as in ABA); this
+// is the body of wave W.  A subtree hands its force (6 scalars) to its trunk parent through
+// an LDS slot (xs); the trunk's tau stays in registers until every wave has read its a.
+// (Humanoid, 50,021 rows: 34.6 us with one wave, the serial walk of one tile per SIMD; 24
+// with four, 37 KB and four workgroups per CU.)
+constexpr int kRneaSlot = 6;
+template<class TP, class S, int kU = kStageU, int G = 1, int W = 0>
 __device__ __forceinline__ void rneaTile(const S* __restrict__ mc_in, int64_t B, int64_t b0, CView<S> gq,
-                                         CView<S> gv, CView<S> ga, View<S> gtau, S* __restrict__ lds) {
+                                         CView<S> gv, CView<S> ga, View<S> gtau, S* __restrict__ lds,
+                                         S* __restrict__ xs = nullptr) {
   using C = DynCfg<TP, S>;
   constexpr auto& T = TP::T;
   constexpr int NJ = C::NJ, NQ = C::NQ, NV = C::NV;
   S* sq = lds;
   S* sv = lds + NQ * kPitch;
   S* sa = lds + (NQ + NV) * kPitch;  // a in, tau out
+  constexpr WaveSplit<TP, G> WS{};
   const int nb = (int)(B - b0 < kTile ? B - b0 : kTile);
-  stageIn<NQ, S, kU>(sq, gq, b0, nb);
-  stageIn<NV, S, kU>(sv, gv, b0, nb);
-  stageIn<NV, S, kU>(sa, ga, b0, nb);
+  if constexpr (W == 0) stageIn<NQ, S, kU>(sq, gq, b0, nb);
+  if constexpr (W == 1 % G) stageIn<NV, S, kU>(sv, gv, b0, nb);
+  if constexpr (W == 2 % G) stageIn<NV, S, kU>(sa, ga, b0, nb);
   __syncthreads();
   const int L = laneId();
   const Mot<S> a0 = mcGravityNeg(mc_in, mcGravity<NJ, NV>());
 
   Mot<S> vj[NJ], aj[NJ];
   Frc<S> fj[NJ];
-  S sn[NJ], cs[NJ];
+  S sn[NJ], cs[NJ], trunk[NV];
+  auto putTau = [&](auto J, auto K, S x) {  // dof K of joint J
+    constexpr int j = decltype(J)::value, k = decltype(K)::value;
+    if constexpr (G > 1 && WS.owner[j] < 0) trunk[k] = x;
+    else sa[k * kPitch + L] = x;
+  };
 
   static_for<0, T.nev>([&](auto E) {
     constexpr int e = E;
+    constexpr int i = TP::T.evJoint[e];
+    if constexpr (WS.runs(i, W)) {
     stepFence();
     const S* __restrict__ mc = stepConsts(mc_in);
-    constexpr int i = TP::T.evJoint[e];
     constexpr int p = TP::T.parent[i];
     constexpr int ty = TP::T.type[i];
     constexpr int iq = TP::T.iq[i], iv = TP::T.iv[i];
@@ -102,34 +116,71 @@ __device__ __forceinline__ void rneaTile(const S* __restrict__ mc_in, int64_t B,
       pinAll<S>(fj[i]);
       if constexpr (ty != JT_FF) pin(sn[i], cs[i]);
     } else {
+      if constexpr (G > 1 && WS.ldsIn[i]) {
+        // subtrees of other waves (fixed order: identical in every wave)
+        __syncthreads();
+        static_for<1, NJ>([&](auto Cc) {
+          constexpr int c = Cc;
+          if constexpr (TP::T.parent[c] == i && WS.slot[c] >= 0) {
+            const S* x = xs + WS.slot[c] * kRneaSlot * kTile + L;
+            fj[i] = fj[i] + Frc<S>{{x[0], x[kTile], x[2 * kTile]}, {x[3 * kTile], x[4 * kTile], x[5 * kTile]}};
+          }
+        });
+      }
+      auto toParent = [&](const Frc<S>& f) {
+        if constexpr (G > 1 && WS.slot[i] >= 0) {
+          S* x = xs + WS.slot[i] * kRneaSlot * kTile + L;
+          x[0] = f.l.x;
+          x[kTile] = f.l.y;
+          x[2 * kTile] = f.l.z;
+          x[3 * kTile] = f.a.x;
+          x[4 * kTile] = f.a.y;
+          x[5 * kTile] = f.a.z;
+        } else {
+          fj[p] = fj[p] + f;
+        }
+      };
       if constexpr (ty == JT_FF) {
         const S f6[6] = {fj[i].l.x, fj[i].l.y, fj[i].l.z, fj[i].a.x, fj[i].a.y, fj[i].a.z};
-#pragma unroll
-        for (int k = 0; k < 6; ++k) {
+        static_for<0, 6>([&](auto K) {
+          constexpr int k = K;
           const S arm = mc[mcArmature<NJ>() + iv + k];
-          sa[(iv + k) * kPitch + L] = f6[k] + arm * sa[(iv + k) * kPitch + L];
-        }
+          if constexpr (WS.writer(i) == W) putTau(IC<i>{}, IC<iv + k>{}, f6[k] + arm * sa[(iv + k) * kPitch + L]);
+        });
         if constexpr (p > 0) {
           S q7[7];
 #pragma unroll
           for (int k = 0; k < 7; ++k) q7[k] = sq[(iq + k) * kPitch + L];
           const Xform<S> X = freeflyerX(mc, i, q7, false);
-          fj[p] = fj[p] + act(X, fj[i]);
+          toParent(act(X, fj[i]));
         }
       } else {
         constexpr int ax = ty - JT_RX;
         const S arm = mc[mcArmature<NJ>() + iv];
-        sa[iv * kPitch + L] = comp(fj[i], 3 + ax) + arm * sa[iv * kPitch + L];
+        if constexpr (WS.writer(i) == W)
+          putTau(IC<i>{}, IC<iv>{}, comp(fj[i], 3 + ax) + arm * sa[iv * kPitch + L]);
         if constexpr (p > 0) {
           const Xform<S> X = revoluteX(mc, i, ax, sn[i], cs[i]);
-          fj[p] = fj[p] + act(X, fj[i]);
-          pinAll<S>(fj[p]);
+          toParent(act(X, fj[i]));
+          if constexpr (WS.slot[i] < 0) pinAll<S>(fj[p]);
         }
       }
     }
+    }
   });
   __syncthreads();
-  stageOut<NV, S, kU>(sa, gtau, b0, nb);
+  if constexpr (G > 1) {
+    static_for<1, NJ>([&](auto J) {
+      constexpr int j = J;
+      if constexpr (WS.owner[j] < 0 && WS.writer(j) == W)
+        static_for<0, TP::T.nvj[j]>([&](auto K) {
+          constexpr int k = TP::T.iv[j] + int(K);
+          sa[k * kPitch + L] = trunk[k];
+        });
+    });
+    __syncthreads();
+  }
+  stageOut<NV, S, kU, G, W>(sa, gtau, b0, nb);
 }
 
 template<class TP, class S>
@@ -138,6 +189,25 @@ __global__ __launch_bounds__(64) void k_rnea(const S* __restrict__ mc, int64_t B
   __shared__ S lds[dynLdsRows<TP>() * kPitch];
   // a single wave stages the whole tile: 16 loads in flight per lane
   rneaTile<TP, S, 2 * kStageU>(mc, B, int64_t(blockIdx.x) * kTile, gq, gv, ga, gtau, lds);
+}
+
+// G waves per tile, split by subtrees
+template<class TP, int G> constexpr int rneaWavesLdsBytes() {
+  constexpr WaveSplit<TP, G> WS{};
+  return (dynLdsRows<TP>() * kPitch + (WS.nslots > 0 ? WS.nslots : 1) * kRneaSlot * kTile) * 4;
+}
+template<class TP, class S, int G>
+__global__ __launch_bounds__(64 * G) void k_rnea_waves(const S* __restrict__ mc, int64_t B, CView<S> gq, CView<S> gv,
+                                                       CView<S> ga, View<S> gtau) {
+  constexpr WaveSplit<TP, G> WS{};
+  __shared__ S lds[dynLdsRows<TP>() * kPitch];
+  __shared__ S xs[(WS.nslots > 0 ? WS.nslots : 1) * kRneaSlot * kTile];
+  const int w = (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  static_for<0, G>([&](auto Wc) {
+    constexpr int W = Wc;
+    if (w == W)
+      rneaTile<TP, S, kStageU, G, W>(mc, B, int64_t(blockIdx.x) * kTile, gq, gv, ga, gtau, lds, xs);
+  });
 }
 
 // ---------------------------------------------------------------------------------------
@@ -339,7 +409,7 @@ __device__ __forceinline__ void abaTile(const S* __restrict__ mc_in, int64_t B, 
     }
   });
   __syncthreads();
-  if (W == 0) stageOut<NV, S, kU>(so, gddq, b0, nb);
+  stageOut<NV, S, kU, G, W>(so, gddq, b0, nb);
 }
 
 template<class TP, class S>

@@ -146,7 +146,8 @@ __device__ __forceinline__ void stageIn(S* __restrict__ lds, CView<S> g, int64_t
     });
   }
 }
-template<int R, class S, int kU = kStageU>
+// (G > 1: the part of wave W of the G that share the tile, every G-th batch of stores)
+template<int R, class S, int kU = kStageU, int G = 1, int W = 0>
 __device__ __forceinline__ void stageOut(const S* __restrict__ lds, View<S> g, int64_t b0, int nb) {
   const int t = laneId();
   if constexpr (kU == 1) {  // compact loop: one row in flight
@@ -165,6 +166,7 @@ __device__ __forceinline__ void stageOut(const S* __restrict__ lds, View<S> g, i
   }
   if (g.rs == 1) {
     static_for<0, (R + kStageU - 1) / kStageU>([&](auto I) {
+      if constexpr (int(I) % G != W) return;
       constexpr int e0 = int(I) * kStageU * kTile;
       S x[kStageU];
       static_for<0, kStageU>([&](auto U) {
@@ -181,6 +183,7 @@ __device__ __forceinline__ void stageOut(const S* __restrict__ lds, View<S> g, i
     });
   } else {
     static_for<0, (R + kStageU - 1) / kStageU>([&](auto I) {
+      if constexpr (int(I) % G != W) return;
       constexpr int k0 = int(I) * kStageU;
       S x[kStageU];
       static_for<0, kStageU>([&](auto U) {
