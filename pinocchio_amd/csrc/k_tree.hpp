@@ -24,7 +24,7 @@
 
 namespace rbd {
 constexpr int kTreeT = 8;            // configurations per workgroup: 8 workers per wave
-constexpr int kTreeMaxThreads = 1024;
+constexpr int kTreeMaxThreads = 512;
 
 // Device tables of one model's tree: 16-bit entries, staged in LDS by every workgroup.
 // The strictly upper entries of the tree pattern are packed by rows: the dofs below dof r
@@ -823,7 +823,8 @@ __global__ __launch_bounds__(kTreeMaxThreads) void t_dsolve(TProg g, int64_t B, 
 // One workgroup's sweep is some 20 phases of short work for its few workers per level: two
 // waves and a small tile leave room for several workgroups per CU.
 // ---------------------------------------------------------------------------------------
-constexpr int kTreeDynC = 23;       // staged constants: placement, mass, lever, inertia
+constexpr int kTreeDynThreads = 128;  // a level has few joints; 16 workers
+constexpr int kTreeDynC = 23;         // staged constants: placement, mass, lever, inertia
 constexpr int kTreeRneaJnt = 25, kTreeAbaJnt = 53;
 template<class S> size_t treeDynLds(const TProg& g, int rec) {
   return (size_t)((g.nTabDyn + 7) & ~7) * 2 +
@@ -876,7 +877,7 @@ __device__ __forceinline__ void treeDynOut(const S* so, View<S> g, int R, int64_
   }
 }
 template<class S>
-__global__ __launch_bounds__(kTreeMaxThreads) void t_rnea(TProg g, const S* __restrict__ mc, int64_t B, CView<S> gq,
+__global__ __launch_bounds__(kTreeDynThreads) void t_rnea(TProg g, const S* __restrict__ mc, int64_t B, CView<S> gq,
                                                           CView<S> gv, CView<S> ga, View<S> gtau) {
   extern __shared__ __align__(16) unsigned char t_lds[];
   const int64_t b0 = treeTile() * kTreeT;
@@ -935,7 +936,7 @@ __global__ __launch_bounds__(kTreeMaxThreads) void t_rnea(TProg g, const S* __re
 }
 
 template<class S>
-__global__ __launch_bounds__(kTreeMaxThreads) void t_aba(TProg g, const S* __restrict__ mc, int64_t B, CView<S> gq,
+__global__ __launch_bounds__(kTreeDynThreads) void t_aba(TProg g, const S* __restrict__ mc, int64_t B, CView<S> gq,
                                                          CView<S> gv, CView<S> gt, View<S> gddq) {
   extern __shared__ __align__(16) unsigned char t_lds[];
   const int64_t b0 = treeTile() * kTreeT;

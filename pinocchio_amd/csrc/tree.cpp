@@ -261,8 +261,6 @@ template<class S> bool treeMinv(hipStream_t st, GM m, const S* mc, int64_t B, CV
   return true;
 }
 
-// RNEA and ABA: a level has few joints; 16 workers
-constexpr unsigned kTreeDynThreads = 128;
 template<class S>
 bool treeRnea(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> tau) {
   const TProg* g = prog(m);
