@@ -206,7 +206,7 @@ void gRneaD(hipStream_t st, GM g, const S* mc, int64_t B, CView<S> q, CView<S> v
 }
 template<class S>
 void gKin(hipStream_t st, GM g, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> oM, View<S> vo,
-          View<S> ao, View<S> J) {
+          View<S> ao, View<S> J, const KinMask&) {
   if (kinRows(oM, vo, ao, J))
     RBD_G_LAUNCH(g_kin_rows, S, kinLane<S>(g), B, progOf(g), mc, B, q, v, a, oM, vo, ao, J);
   else

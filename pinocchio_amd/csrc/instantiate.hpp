@@ -158,13 +158,36 @@ void launchAbaDSolve(hipStream_t st, GM, int64_t B, CView<S> U, CView<S> D, View
 }
 
 
+// a subtree split of the kinematics over four waves
+template<class TP> constexpr bool kinSplitPays() {
+  constexpr WaveSplit<TP, 4> WS{};
+  int trunk = 0, busiest = 0;
+  for (int j = 1; j < TP::NJ; ++j) trunk += WS.owner[j] < 0 ? 1 : 0;
+  for (int k = 0; k < 4; ++k) busiest = WS.load[k] > busiest ? WS.load[k] : busiest;
+  return 5 * (trunk + busiest) <= 3 * (TP::NJ - 1);
+}
+template<class TP, class S, int G>
+void launchKinWaves(hipStream_t st, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> oM,
+                    View<S> vo, View<S> ao, View<S> J, const KinMask& want) {
+  if (kinRows(oM, vo, ao, J))
+    hipLaunchKernelGGL((k_kin<TP, S, true, G>), dim3(gridFor(B)), dim3(kTile * G), 0, st, mc, B, q, v, a, oM, vo, ao,
+                       J, want);
+  else
+    hipLaunchKernelGGL((k_kin<TP, S, false, G>), dim3(gridFor(B)), dim3(kTile * G), 0, st, mc, B, q, v, a, oM, vo, ao,
+                       J, want);
+}
+// Four waves per tile up to one tile per CU, or two when only the Jacobian is written; beyond
+// that the stores bound the kernel and one wave's come in better order (humanoid, us per
+// call, one wave / four: placements and motions 56 / 36 at 16,384, 60 / 69 at 30,011, FP64
+// rows 215 / 256 at 65,536; Jacobian 33 / 24, 34 / 28, rows 45 / 49 at 65,536).
 template<class TP, class S>
 void launchKin(hipStream_t st, GM, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> oM, View<S> vo,
-               View<S> ao, View<S> J) {
-  if (kinRows(oM, vo, ao, J))
-    hipLaunchKernelGGL((k_kin<TP, S, true>), dim3(gridFor(B)), dim3(kTile), 0, st, mc, B, q, v, a, oM, vo, ao, J);
-  else
-    hipLaunchKernelGGL((k_kin<TP, S, false>), dim3(gridFor(B)), dim3(kTile), 0, st, mc, B, q, v, a, oM, vo, ao, J);
+               View<S> ao, View<S> J, const KinMask& want) {
+  if constexpr (kinSplitPays<TP>()) {
+    if (B <= (int64_t)256 * kTile * (oM.p || vo.p ? 1 : 2))
+      return launchKinWaves<TP, S, 4>(st, mc, B, q, v, a, oM, vo, ao, J, want);
+  }
+  launchKinWaves<TP, S, 1>(st, mc, B, q, v, a, oM, vo, ao, J, want);
 }
 
 template<class TP, class S>

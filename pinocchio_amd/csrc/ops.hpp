@@ -35,11 +35,18 @@ template<class S>
 using LaunchAbaDSolve = void (*)(hipStream_t, GM, int64_t B, CView<S> U, CView<S> D, View<S> Xq, View<S> Xv,
                                  View<S> Minv, int jobBegin);
 
+// Joints and dofs whose outputs are wanted (bit i: joint i's placement and motions; the
+// Jacobian columns of joint i's dofs): the constraint rows need those of their joints only.
+struct KinMask {
+  uint64_t joints = ~0ull, columns = ~0ull;
+};
+
 // forward kinematics / joint Jacobians: outputs placements, local velocities and
-// accelerations, WORLD Jacobian columns (any may be null)
+// accelerations, WORLD Jacobian columns (any may be null); want: the joints whose outputs
+// are needed (the run-time-topology kernels write all)
 template<class S>
 using LaunchKin = void (*)(hipStream_t, GM, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> oM,
-                           View<S> vo, View<S> ao, View<S> J);
+                           View<S> vo, View<S> ao, View<S> J, const KinMask& want);
 
 // forward dynamics under J ddq + gamma = 0 from the FP64 tree factor of M and nle: ddq,
 // lambda; mode 1: impulse dynamics with v_before in `tau` (nle and gamma unused); mode 2:

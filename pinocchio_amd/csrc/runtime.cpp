@@ -732,7 +732,7 @@ void kinCall(rbd_ctx* ctx, const rbd_model* m, int64_t B, const void* q, int64_t
   reinterpret_cast<LaunchKin<S>>(launch)(ctx->stream, m->gen.get(), mc, B, CView<S>{dq, vq.rs, vq.bs}, CView<S>{dv, vv.rs, vv.bs},
                                         CView<S>{da, va.rs, va.bs}, View<S>{dM, vM.rs, vM.bs},
                                         View<S>{dvo, vva.rs, vva.bs}, View<S>{dao, vva.rs, vva.bs},
-                                        View<S>{dJ, vJ.rs, vJ.bs});
+                                        View<S>{dJ, vJ.rs, vJ.bs}, KinMask{});
   finishCall(ctx, flags, st);
 }
 }  // namespace
@@ -1121,7 +1121,7 @@ void framesCall(rbd_ctx* ctx, const rbd_model* m, int64_t B, const void* q, int6
   if constexpr (f32) mc = m->mc32;
   else mc = m->mc64;
   reinterpret_cast<LaunchKin<S>>(launch)(ctx->stream, m->gen.get(), mc, B, CView<S>{dq, vq.rs, vq.bs}, CView<S>{}, CView<S>{},
-                                        View<S>{wO, B, 1}, View<S>{}, View<S>{}, View<S>{wJ, B, 1});
+                                        View<S>{wO, B, 1}, View<S>{}, View<S>{}, View<S>{wJ, B, 1}, KinMask{});
   hipLaunchKernelGGL(k_frames<S>, dim3((unsigned)((B + 255) / 256), (unsigned)nf), dim3(256), 0, ctx->stream, B, nv,
                      dpar, dpl, dsup, CView<S>{wO, B, 1}, CView<S>{wJ, B, 1}, rf, View<S>{dM, vM.rs, vM.bs},
                      View<S>{dJ, vJ.rs, vJ.bs});
@@ -1173,7 +1173,7 @@ void frameMotionsCall(rbd_ctx* ctx, const rbd_model* m, int64_t B, const void* q
   else mc = m->mc64;
   reinterpret_cast<LaunchKin<S>>(launch)(ctx->stream, m->gen.get(), mc, B, CView<S>{dq, vq.rs, vq.bs},
                                         CView<S>{dv, vv.rs, vv.bs}, CView<S>{da, va.rs, va.bs}, View<S>{wO, B, 1},
-                                        View<S>{wV, B, 1}, View<S>{wA, B, 1}, View<S>{});
+                                        View<S>{wV, B, 1}, View<S>{wA, B, 1}, View<S>{}, KinMask{});
   hipLaunchKernelGGL(k_frame_motions<S>, dim3((unsigned)((B + 255) / 256), (unsigned)nf), dim3(256), 0, ctx->stream,
                      B, dpar, dpl, CView<S>{wO, B, 1}, CView<S>{wV, B, 1}, CView<S>{wA, B, 1}, rf,
                      View<S>{dvf, vo.rs, vo.bs}, View<S>{daf, vo.rs, vo.bs}, View<S>{dacf, vo.rs, vo.bs});
@@ -1219,7 +1219,7 @@ void jacobianDotCall(rbd_ctx* ctx, const rbd_model* m, int64_t B, const void* q,
   else mc = m->mc64;
   reinterpret_cast<LaunchKin<S>>(launch)(ctx->stream, m->gen.get(), mc, B, CView<S>{dq, vq.rs, vq.bs},
                                         CView<S>{dv, vv.rs, vv.bs}, CView<S>{}, View<S>{wO, B, 1}, View<S>{wV, B, 1},
-                                        View<S>{}, View<S>{wJ, B, 1});
+                                        View<S>{}, View<S>{wJ, B, 1}, KinMask{});
   hipLaunchKernelGGL(k_jacobian_dot<S>, dim3((unsigned)((B + 255) / 256), (unsigned)nv), dim3(256), 0, ctx->stream, B,
                      (const int32_t*)dtab, CView<S>{wO, B, 1}, CView<S>{wV, B, 1}, CView<S>{wJ, B, 1},
                      View<S>{ddJ, vd.rs, vd.bs}, View<S>{dJo, vJ.rs, vJ.bs});
@@ -1278,7 +1278,7 @@ void frameJacobianDotCall(rbd_ctx* ctx, const rbd_model* m, int64_t B, const voi
   else mc = m->mc64;
   reinterpret_cast<LaunchKin<S>>(launch)(ctx->stream, m->gen.get(), mc, B, CView<S>{dq, vq.rs, vq.bs},
                                         CView<S>{dv, vv.rs, vv.bs}, CView<S>{}, View<S>{wO, B, 1}, View<S>{wV, B, 1},
-                                        View<S>{}, View<S>{wJ, B, 1});
+                                        View<S>{}, View<S>{wJ, B, 1}, KinMask{});
   const unsigned gb = (unsigned)((B + 255) / 256);
   hipLaunchKernelGGL(k_jacobian_dot<S>, dim3(gb, (unsigned)nv), dim3(256), 0, ctx->stream, B, ddof, CView<S>{wO, B, 1},
                      CView<S>{wV, B, 1}, CView<S>{wJ, B, 1}, View<S>{wD, B, 1}, View<S>{});
@@ -1433,6 +1433,17 @@ int constraintTable(const rbd_model* m, int ncon, const rbd_rigid_constraint* co
   return nrows;
 }
 
+// what the rows of the constraints read of the kinematics
+KinMask constraintMask(const rbd_model* m, int ncon, const rbd_rigid_constraint* cons) {
+  KinMask k{0, 0};
+  for (int c = 0; c < ncon; ++c)
+    for (int j : {cons[c].joint1_id, cons[c].joint2_id}) {
+      k.joints |= 1ull << (j & 63);
+      for (int a = j; a > 0; a = m->parents[a]) k.columns |= 1ull << (a & 63);
+    }
+  return k;
+}
+
 template<class S>
 void cdCall(rbd_ctx* ctx, const rbd_model* m, int64_t B, const void* q, int64_t ldq, const void* v, int64_t ldv,
             const void* tau, int64_t ldtau, int ncon, const rbd_rigid_constraint* cons, const rbd_proximal_settings& ps,
@@ -1487,9 +1498,9 @@ void cdCall(rbd_ctx* ctx, const rbd_model* m, int64_t B, const void* q, int64_t 
   hipLaunchKernelGGL(k_fill_zero<S>, dim3(1), dim3(64), 0, ctx->stream, wZ, (int64_t)1);
   const auto kin = f32 ? (LaunchKin<S>)o.kin_f32 : (LaunchKin<S>)o.kin_f64;
   kin(ctx->stream, m->gen.get(), mc, B, cq, cv, zero, View<S>{wO, B, 1}, View<S>{wV, B, 1}, View<S>{wA, B, 1},
-      View<S>{wJw, B, 1});
-  hipLaunchKernelGGL(k_contact_terms<S>, dim3((unsigned)((B + 255) / 256)), dim3(256), 0, ctx->stream, B, nv, ncon,
-                     nrows, dtab, dsup, CView<S>{wO, B, 1}, CView<S>{wV, B, 1}, CView<S>{wA, B, 1},
+      View<S>{wJw, B, 1}, constraintMask(m, ncon, cons));
+  hipLaunchKernelGGL(k_contact_terms<S>, dim3((unsigned)((B + 63) / 64), (unsigned)ncon, kContactParts), dim3(64), 0,
+                     ctx->stream, B, nv, nrows, dtab, dsup, CView<S>{wO, B, 1}, CView<S>{wV, B, 1}, CView<S>{wA, B, 1},
                      CView<S>{wJw, B, 1}, View<S>{wJc, B, 1}, View<S>{wG, B, 1});
   if constexpr (f32) {
     o.crba_f32(ctx->stream, m->gen.get(), mc, B, cq, View<S>{wM, B, 1}, 0);
@@ -1563,9 +1574,9 @@ void constraintMatrixCall(rbd_ctx* ctx, const rbd_model* m, int64_t B, const voi
   hipLaunchKernelGGL(k_fill_zero<S>, dim3(1), dim3(64), 0, ctx->stream, wZ, (int64_t)1);
   const auto kin = f32 ? (LaunchKin<S>)o.kin_f32 : (LaunchKin<S>)o.kin_f64;
   kin(ctx->stream, m->gen.get(), mc, B, cq, zero, zero, View<S>{wO, B, 1}, View<S>{wV, B, 1}, View<S>{wA, B, 1},
-      View<S>{wJw, B, 1});
-  hipLaunchKernelGGL(k_contact_terms<S>, dim3((unsigned)((B + 255) / 256)), dim3(256), 0, ctx->stream, B, nv, ncon,
-                     nrows, dtab, dsup, CView<S>{wO, B, 1}, CView<S>{wV, B, 1}, CView<S>{wA, B, 1},
+      View<S>{wJw, B, 1}, constraintMask(m, ncon, cons));
+  hipLaunchKernelGGL(k_contact_terms<S>, dim3((unsigned)((B + 63) / 64), (unsigned)ncon, kContactParts), dim3(64), 0,
+                     ctx->stream, B, nv, nrows, dtab, dsup, CView<S>{wO, B, 1}, CView<S>{wV, B, 1}, CView<S>{wA, B, 1},
                      CView<S>{wJw, B, 1}, View<S>{wJc, B, 1}, View<S>{wGm, B, 1});
   if constexpr (f32) {
     o.crba_f32(ctx->stream, m->gen.get(), mc, B, cq, View<S>{wM, B, 1}, 0);
