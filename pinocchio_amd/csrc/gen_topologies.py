@@ -40,10 +40,17 @@ WAVE_KERNELS = {
             ("k_rnea_waves", "float", _VEC3.format(s="float"), (4,)),
             ("k_rnea_waves", "double", _VEC3.format(s="double"), (4,))],
     "rnead": [("k_rnead", "float", _RNEAD, (4,))],
+    "crba": [("k_crba_waves", s, f"const {s}*, int64_t, CView<{s}>, View<{s}>, int", (4,)) for s in ("float", "double")],
+    "chol": [("k_chol_waves", f"{i}, {c}", f"int64_t, CView<{i}>, View<{c}>, View<{c}>", (4,))
+             for i, c in (("float", "double"), ("double", "double"), ("float", "float"))],
 }
+# unit name suffix per scalar (or input and factor scalar)
+SCALAR_TAG = {"float": "", "double": "d", "float, double": "fd", "double, double": "dd", "float, float": "ff"}
 WAVE_TAG = {"k_rnea_waves": "rnea_"}  # units of a family's second multi-wave kernel
 WAVE_COND = {"k_aba_waves": "abaSplitPaysFor<Topo_{name}, {sc}, {g}>()",
              "k_rnea_waves": "rneaSplitPaysFor<Topo_{name}, {sc}, {g}>()",
+             "k_crba_waves": "crbaSplitPaysFor<Topo_{name}, {sc}, {g}>()",
+             "k_chol_waves": "cholSplitPaysFor<Topo_{name}, {sc}, {g}>()",
              "k_rnead": "rneadSplitPays<Topo_{name}, {g}>()"}
 
 DYN = ["dyn", "kin"]
@@ -170,7 +177,7 @@ def main(out_dir=None, robots=""):
             for k, sc, sig, gs in WAVE_KERNELS.get(fam, []):
                 for g in gs:
                     cond = WAVE_COND[k].format(name=name, g=g, sc=sc)
-                    tag = f"{WAVE_TAG.get(k, '')}w{g}" + ("" if sc == "float" else "d")
+                    tag = f"{WAVE_TAG.get(k, '')}w{g}" + SCALAR_TAG[sc]
                     _write(os.path.join(out_dir, f"inst_{name}_{fam}_{tag}.hip"),
                            "// generated by gen_topologies.py -- do not edit\n"
                            "#include \"../instantiate.hpp\"\nnamespace rbd {\n"

@@ -108,21 +108,56 @@ void launchAba(hipStream_t st, GM, const S* mc, int64_t B, CView<S> q, CView<S> 
     hipLaunchKernelGGL((k_aba<TP, S>), dim3(gridFor(B)), dim3(kTile), 0, st, mc, B, q, v, tau, out);
   }
 }
-// CRBA: two waves per tile (output emission split) keep two waves resident per SIMD at
-// large batches
+// the tree splits over four waves (the tests above without an algorithm's LDS)
+template<class TP> constexpr bool treeSplits() {
+  constexpr WaveSplit<TP, 4> WS{};
+  int trunk = 0, busiest = 0;
+  for (int j = 1; j < TP::NJ; ++j) trunk += WS.owner[j] < 0 ? 1 : 0;
+  for (int k = 0; k < 4; ++k) busiest = WS.load[k] > busiest ? WS.load[k] : busiest;
+  return 5 * (trunk + busiest) <= 3 * (TP::NJ - 1);
+}
+template<class TP, class S, int G> constexpr bool crbaSplitPaysFor() {
+  return treeSplits<TP>() && crbaWavesLdsBytes<TP, G>() / 4 * (int)sizeof(S) <= 160 * 1024;
+}
+template<class TP, class SIN, class SC, int G> constexpr bool cholSplitPaysFor() {
+  return treeSplits<TP>() && cholWavesLdsBytes<TP, SC, G>() <= 160 * 1024;
+}
+// CRBA: up to one tile per CU four waves split the tree (humanoid, 16,384: 49 us of kernel on
+// two waves, 22 on four writing the factorisation's entries); beyond, two waves per tile
+// (output emission split) keep two waves resident per SIMD
 template<class TP, class S>
 void launchCrba(hipStream_t st, GM, const S* mc, int64_t B, CView<S> q, View<S> M, int upper) {
+  if constexpr (crbaSplitPaysFor<TP, S, 4>()) {
+    if (B <= 256 * kTile) {
+      hipLaunchKernelGGL((k_crba_waves<TP, S, 4>), dim3(gridFor(B)), dim3(kTile * 4), 0, st, mc, B, q, M, upper);
+      return;
+    }
+  }
   if (TP::NJ <= 3)
     hipLaunchKernelGGL((k_crba<TP, S, 1>), dim3(gridFor(B)), dim3(kTile), 0, st, mc, B, q, M, upper);
   else
     hipLaunchKernelGGL((k_crba<TP, S, 2>), dim3(gridFor(B)), dim3(kTile * 2), 0, st, mc, B, q, M, upper);
 }
+// four waves per tile up to one tile per CU (humanoid, 16,384: FP64 27 us of kernel, 15 on
+// four; FP32 staged 22, 12)
+template<class TP, class SIN, class SC>
+bool launchCholWaves(hipStream_t st, int64_t B, CView<SIN> M, View<SC> U, View<SC> D) {
+  if constexpr (cholSplitPaysFor<TP, SIN, SC, 4>()) {
+    if (B <= 256 * kTile) {
+      hipLaunchKernelGGL((k_chol_waves<TP, SIN, SC, 4>), dim3(gridFor(B)), dim3(kTile * 4), 0, st, B, M, U, D);
+      return true;
+    }
+  }
+  return false;
+}
 template<class TP, class S> void launchChol(hipStream_t st, GM, int64_t B, CView<S> M, View<double> U, View<double> D) {
+  if (launchCholWaves<TP, S, double>(st, B, M, U, D)) return;
   hipLaunchKernelGGL((k_chol<TP, S, double>), dim3(gridFor(B)), dim3(kTile), 0, st, B, M, U, D);
 }
 // FP32 factor (ABA derivatives, computeMinverse): M staged into LDS first when the batch
 // leaves about two tiles per CU or fewer
 template<class TP> void launchChol32(hipStream_t st, GM, int64_t B, CView<float> M, View<float> U, View<float> D) {
+  if (launchCholWaves<TP, float, float>(st, B, M, U, D)) return;
   const bool staged = (B + kTile - 1) / kTile <= 512;
   if (staged && cholStagedLdsBytes<TP, float>() <= 160 * 1024)
     hipLaunchKernelGGL((k_chol_staged<TP, float, float>), dim3(gridFor(B)), dim3(kTile), 0, st, B, M, U, D);
@@ -158,14 +193,6 @@ void launchAbaDSolve(hipStream_t st, GM, int64_t B, CView<S> U, CView<S> D, View
 }
 
 
-// a subtree split of the kinematics over four waves
-template<class TP> constexpr bool kinSplitPays() {
-  constexpr WaveSplit<TP, 4> WS{};
-  int trunk = 0, busiest = 0;
-  for (int j = 1; j < TP::NJ; ++j) trunk += WS.owner[j] < 0 ? 1 : 0;
-  for (int k = 0; k < 4; ++k) busiest = WS.load[k] > busiest ? WS.load[k] : busiest;
-  return 5 * (trunk + busiest) <= 3 * (TP::NJ - 1);
-}
 template<class TP, class S, int G>
 void launchKinWaves(hipStream_t st, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> oM,
                     View<S> vo, View<S> ao, View<S> J, const KinMask& want) {
@@ -183,7 +210,7 @@ void launchKinWaves(hipStream_t st, const S* mc, int64_t B, CView<S> q, CView<S>
 template<class TP, class S>
 void launchKin(hipStream_t st, GM, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> oM, View<S> vo,
                View<S> ao, View<S> J, const KinMask& want) {
-  if constexpr (kinSplitPays<TP>()) {
+  if constexpr (treeSplits<TP>()) {
     if (B <= (int64_t)256 * kTile * (oM.p || vo.p ? 1 : 2))
       return launchKinWaves<TP, S, 4>(st, mc, B, q, v, a, oM, vo, ao, J, want);
   }

@@ -63,8 +63,10 @@ template<class S> __device__ __forceinline__ void stMat(View<S> g, int64_t b, in
 }
 
 // ---------------------------------------------------------------------------------------
-// CRBA: M(q), symmetric (or upper row blocks only), armature on the diagonal
+// CRBA: M(q), symmetric (or upper row blocks only), armature on the diagonal.  upperOnly ==
+// kMassPattern: the upper structural entries alone, all that the factorisation reads.
 // ---------------------------------------------------------------------------------------
+constexpr int kMassPattern = 2;
 // G > 1: G waves share the tile; all run the forward pass and the composite-inertia
 // accumulation (cheap), and joint i's entries are computed and stored by wave
 // EmitGroups<TP, G>::grp[i] only, so the store-heavy emission is spread over more waves.
@@ -133,7 +135,7 @@ __device__ __forceinline__ void crbaTile(const S* __restrict__ mc_in, int64_t B,
           if (r == c) m += mc[mcArmature<NJ>() + c];
           if (live) {
             stMat(gM, b, NV, r, c, m);
-            if (r != c) stMat(gM, b, NV, c, r, m);
+            if (r != c && upperOnly != kMassPattern) stMat(gM, b, NV, c, r, m);
           }
         }
         // ancestors
@@ -161,7 +163,7 @@ __device__ __forceinline__ void crbaTile(const S* __restrict__ mc_in, int64_t B,
     }
   });
   // structural zeros (upper triangle only in upper-only mode)
-  if (live) {
+  if (live && upperOnly != kMassPattern) {
     static_for<0, NV>([&](auto C) {
       static_for<0, NV>([&](auto R) {
         if constexpr (!CrbaPattern<TP>::nz(R, C)) {
@@ -178,6 +180,147 @@ __global__ __launch_bounds__(64 * G) void k_crba(const S* __restrict__ mc_in, in
   __shared__ S sq[TP::T.nq * kPitch];
   const int w = G > 1 ? (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
   crbaTile<TP, S, G>(mc_in, B, int64_t(blockIdx.x) * kTile, gq, gM, upperOnly, sq, w);
+}
+
+// The same on G waves that split the tree by subtrees (WaveSplit) instead of the emission:
+// with one tile per CU the kernel takes one wave's walk, and a wave of the split walks the
+// trunk and its subtrees only.  A subtree hands its composite inertia (10 scalars) to its
+// trunk parent through an LDS slot; a joint's entries are stored by its owner, the trunk's by
+// wave 0.  This is the body of wave W.
+constexpr int kCrbaSlot = 10;
+template<class TP, int G> constexpr int crbaWavesLdsBytes() {
+  constexpr WaveSplit<TP, G> WS{};
+  return (TP::T.nq * kPitch + (WS.nslots > 0 ? WS.nslots : 1) * kCrbaSlot * kTile) * 4;
+}
+template<class TP, class S, int G, int W>
+__device__ __forceinline__ void crbaSplitTile(const S* __restrict__ mc_in, int64_t B, int64_t b0, CView<S> gq,
+                                              View<S> gM, int upperOnly, S* __restrict__ sq, S* __restrict__ xs) {
+  constexpr auto& T = TP::T;
+  constexpr int NJ = TP::NJ, NQ = T.nq, NV = T.nv;
+  constexpr WaveSplit<TP, G> WS{};
+  const int nb = (int)(B - b0 < kTile ? B - b0 : kTile);
+  constexpr int NQh = (NQ + 1) / 2;  // two waves stage half of q each
+  if constexpr (W == 0) stageIn<NQh>(sq, gq, b0, nb);
+  if constexpr (W == 1) stageIn<NQ - NQh>(sq + NQh * kPitch, CView<S>{gq.p + (int64_t)NQh * gq.rs, gq.rs, gq.bs}, b0, nb);
+  __syncthreads();
+  const int L = laneId();
+  const int64_t b = b0 + L;
+  const bool live = L < nb;
+  const bool lower = upperOnly == 0;
+
+  Xform<S> oM[NJ];
+  CInertia<S> Yacc[NJ];
+
+  static_for<0, T.nev>([&](auto E) {
+    constexpr int e = E;
+    constexpr int i = TP::T.evJoint[e];
+    if constexpr (WS.runs(i, W)) {
+    stepFence();
+    const S* __restrict__ mc = stepConsts(mc_in);
+    constexpr int p = TP::T.parent[i];
+    constexpr int ty = TP::T.type[i];
+    constexpr int iq = TP::T.iq[i], iv = TP::T.iv[i], nvi = TP::T.nvj[i];
+    if constexpr (TP::T.evKind[e] == EV_PRE) {
+      Xform<S> X;
+      if constexpr (ty == JT_FF) {
+        S q7[7];
+#pragma unroll
+        for (int k = 0; k < 7; ++k) q7[k] = sq[(iq + k) * kPitch + L];
+        X = freeflyerX(mc, i, q7, false);
+        X.p = {S(0), S(0), S(0)};  // frame origin at the floating base (see the header)
+      } else {
+        S sn, cs;
+        sincosT(sq[iq * kPitch + L], &sn, &cs);
+        X = revoluteX(mc, i, ty - JT_RX, sn, cs);
+      }
+      if constexpr (p > 0) oM[i] = compose(oM[p], X);
+      else oM[i] = X;
+      pinAll<S>(oM[i]);
+    } else {
+      CInertia<S> Y = worldInertia(mc, i, oM[i]);
+      if constexpr (WS.nReg[i] > 0) cadd(Y, Yacc[i]);
+      if constexpr (WS.ldsIn[i]) {
+        __syncthreads();  // subtrees of other waves (fixed order: identical in every wave)
+        static_for<1, NJ>([&](auto Cc) {
+          constexpr int c = Cc;
+          if constexpr (TP::T.parent[c] == i && WS.slot[c] >= 0) {
+            const S* x = xs + WS.slot[c] * kCrbaSlot * kTile + L;
+            CInertia<S> Yc;
+            S* yc = reinterpret_cast<S*>(&Yc);
+#pragma unroll
+            for (int k = 0; k < 10; ++k) yc[k] = x[k * kTile];
+            cadd(Y, Yc);
+          }
+        });
+      }
+      if constexpr (p > 0) {
+        if constexpr (WS.slot[i] >= 0) {
+          S* x = xs + WS.slot[i] * kCrbaSlot * kTile + L;
+          const S* yc = reinterpret_cast<const S*>(&Y);
+#pragma unroll
+          for (int k = 0; k < 10; ++k) x[k * kTile] = yc[k];
+        } else if constexpr (WS.regIdx[i] == 0) {
+          Yacc[p] = Y;
+        } else {
+          cadd(Yacc[p], Y);
+        }
+      }
+      if constexpr (WS.writer(i) == W) {
+#pragma unroll
+        for (int k = 0; k < nvi; ++k) {
+          const int c = iv + k;
+          const Frc<S> F = cmul(Y, worldAxis<ty>(oM[i], k));
+#pragma unroll
+          for (int k2 = 0; k2 <= k; ++k2) {
+            const int r = iv + k2;
+            S m = dot(worldAxis<ty>(oM[i], k2), F);
+            if (r == c) m += mc[mcArmature<NJ>() + c];
+            if (live) {
+              stMat(gM, b, NV, r, c, m);
+              if (r != c && upperOnly != kMassPattern) stMat(gM, b, NV, c, r, m);
+            }
+          }
+          static_for<1, NJ>([&](auto A) {
+            constexpr int a = A;
+            if constexpr (a != i && TP::T.pos[a] < TP::T.pos[i] && TP::T.pos[a] + TP::T.subsize[a] > TP::T.pos[i]) {
+              constexpr int tya = TP::T.type[a];
+#pragma unroll
+              for (int k2 = 0; k2 < TP::T.nvj[a]; ++k2) {
+                const int r = TP::T.iv[a] + k2;
+                const S m = dot(worldAxis<tya>(oM[a], k2), F);
+                if (live) {
+                  stMat(gM, b, NV, r, c, m);
+                  if (lower) stMat(gM, b, NV, c, r, m);
+                }
+              }
+            }
+          });
+        }
+      }
+    }
+    }
+  });
+  if (live && upperOnly != kMassPattern) {
+    static_for<0, NV>([&](auto C) {
+      static_for<0, NV>([&](auto R) {
+        if constexpr (!CrbaPattern<TP>::nz(R, C) && (int)C % G == W) {
+          if (lower || R <= C) stMat(gM, b, NV, R, C, S(0));
+        }
+      });
+    });
+  }
+}
+template<class TP, class S, int G>
+__global__ __launch_bounds__(64 * G) void k_crba_waves(const S* __restrict__ mc, int64_t B, CView<S> gq, View<S> gM,
+                                                       int upperOnly) {
+  constexpr WaveSplit<TP, G> WS{};
+  __shared__ S sq[TP::T.nq * kPitch];
+  __shared__ S xs[(WS.nslots > 0 ? WS.nslots : 1) * kCrbaSlot * kTile];
+  const int w = (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  static_for<0, G>([&](auto Wc) {
+    constexpr int W = Wc;
+    if (w == W) crbaSplitTile<TP, S, G, W>(mc, B, int64_t(blockIdx.x) * kTile, gq, gM, upperOnly, sq, xs);
+  });
 }
 
 // ---------------------------------------------------------------------------------------
@@ -372,6 +515,136 @@ __global__ __launch_bounds__(64) void k_chol_staged(int64_t B, CView<SIN> gM, Vi
         });
       }
     });
+  });
+}
+
+// The same factorisation on G waves that share a tile (WaveSplit): a wave eliminates the
+// columns of its subtrees, all its entries of M loaded up front, and adds up what they take
+// from the trunk's block; the sums meet in LDS and wave 0 eliminates the trunk.  With one
+// tile per CU the elimination is one wave's chain, and here the longest is a subtree's and
+// the trunk's.  Packed entries and D as k_chol.
+// (Ancestors, packed positions and trunk slots are tables: scanning all pairs at compile
+// time costs minutes per topology.)
+template<class TP, int G> struct CholSplit {
+  static constexpr int NV = TP::T.nv;
+  int n[NV] = {}, base[NV] = {}, anc[NV][NV] = {};  // ancestors of a dof, root first; packed start
+  int touch[NV] = {};   // column that first touches the entries of column c
+  int owner[NV] = {};   // wave of the dof's joint, -1: trunk
+  int pair0[NV] = {};   // trunk column c: slots of its ancestors' entries, then its diagonal
+  int npairs = 0;
+  constexpr CholSplit() {
+    constexpr WaveSplit<TP, G> WS{};
+    int at = 0;
+    for (int c = 0; c < NV; ++c) {
+      const int p = TP::T.dofParent[c];
+      if (p >= 0) {
+        n[c] = n[p] + 1;
+        for (int k = 0; k < n[p]; ++k) anc[c][k] = anc[p][k];
+        anc[c][n[p]] = p;
+      }
+      base[c] = at;
+      at += n[c];
+      touch[c] = CholPattern<TP>::firstTouch(c, c);
+      owner[c] = WS.owner[TP::T.dofJoint[c]];
+      if (owner[c] < 0) {
+        pair0[c] = npairs;
+        npairs += n[c] + 1;
+      }
+    }
+  }
+};
+template<class TP, class SC, int G> constexpr int cholWavesLdsBytes() {
+  constexpr CholSplit<TP, G> CS{};
+  return G * (CS.npairs > 0 ? CS.npairs : 1) * kTile * (int)sizeof(SC);
+}
+template<class TP, class SIN, class SC, int G, int W>
+__device__ __forceinline__ void cholSplitTile(int64_t B, CView<SIN> gM, View<SC> gU, View<SC> gD, SC* __restrict__ xs) {
+  constexpr int NV = TP::T.nv;
+  constexpr CholSplit<TP, G> CS{};
+  const int L = laneId();
+  const int64_t b0 = int64_t(blockIdx.x) * kTile + L;
+  const bool live = b0 < B;
+  const int64_t b = live ? b0 : B - 1;
+  SIN in[NV][NV];  // this wave's entries of M
+  SC A[NV][NV];    // only pattern entries are materialised
+  // entries (r, c) of column c, the diagonal last
+  auto column = [&](auto C, auto f) {
+    constexpr int c = decltype(C)::value;
+    static_for<0, CS.n[c] + 1>([&](auto K) {
+      constexpr int k = K;
+      constexpr int r = k < CS.n[c] ? CS.anc[c][k] : c;
+      f(IC<r>{}, IC<c>{}, IC<k>{});
+    });
+  };
+  auto columnsOf = [&](auto Own, auto f) {
+    constexpr int own = decltype(Own)::value;
+    static_for<0, NV>([&](auto C) {
+      if constexpr (CS.owner[int(C)] == own) column(C, f);
+    });
+  };
+  auto preload = [&](auto R, auto C, auto) {
+    constexpr int r = decltype(R)::value, c = decltype(C)::value;
+    in[r][c] = gM.p[(int64_t)(r + c * NV) * gM.rs + b * gM.bs];
+  };
+  columnsOf(IC<W>{}, preload);
+  if constexpr (W == 0) columnsOf(IC<-1>{}, preload);
+  // columns of owner `own`, last first; a subtree's wave starts the trunk's entries from zero
+  auto eliminate = [&](auto Own) {
+    constexpr int own = decltype(Own)::value;
+    static_for<0, NV>([&](auto JJ) {
+      constexpr int j = NV - 1 - JJ;
+      if constexpr (CS.owner[j] == own) {
+        stepFence();
+        auto first = [&](auto R, auto C, auto) {
+          constexpr int r = decltype(R)::value, c = decltype(C)::value;
+          A[r][c] = SC(in[r][c]);
+        };
+        if constexpr (own >= 0 && CS.touch[j] == j) column(IC<j>{}, first);
+        const SC Dj = A[j][j];
+        const SC Dinv = SC(1) / Dj;
+        if (live) stOut(&gD.p[(int64_t)j * gD.rs + b * gD.bs], Dj);
+        SC Uc[NV];
+        static_for<0, CS.n[j]>([&](auto K) {
+          constexpr int r = CS.anc[j][int(K)];
+          Uc[r] = A[r][j] * Dinv;
+          if (live) stOut(&gU.p[(int64_t)(CS.base[j] + int(K)) * gU.rs + b * gU.bs], Uc[r]);
+        });
+        static_for<0, CS.n[j]>([&](auto K) {
+          constexpr int r2 = CS.anc[j][int(K)];
+          if constexpr (own >= 0 && CS.owner[r2] >= 0 && CS.touch[r2] == j) column(IC<r2>{}, first);
+          column(IC<r2>{}, [&](auto R1, auto, auto) {
+            constexpr int r1 = decltype(R1)::value;
+            A[r1][r2] -= Uc[r1] * A[r2][j];
+          });
+        });
+      }
+    });
+  };
+  columnsOf(IC<-1>{}, [&](auto R, auto C, auto) { A[decltype(R)::value][decltype(C)::value] = SC(0); });
+  eliminate(IC<W>{});
+  columnsOf(IC<-1>{}, [&](auto R, auto C, auto K) {
+    constexpr int r = decltype(R)::value, c = decltype(C)::value;
+    xs[(W * CS.npairs + CS.pair0[c] + decltype(K)::value) * kTile + L] = A[r][c];
+  });
+  __syncthreads();
+  if constexpr (W == 0) {
+    columnsOf(IC<-1>{}, [&](auto R, auto C, auto K) {
+      constexpr int r = decltype(R)::value, c = decltype(C)::value;
+      SC x = SC(in[r][c]);
+#pragma unroll
+      for (int w = 0; w < G; ++w) x += xs[(w * CS.npairs + CS.pair0[c] + decltype(K)::value) * kTile + L];
+      A[r][c] = x;
+    });
+    eliminate(IC<-1>{});
+  }
+}
+template<class TP, class SIN, class SC, int G>
+__global__ __launch_bounds__(64 * G) void k_chol_waves(int64_t B, CView<SIN> gM, View<SC> gU, View<SC> gD) {
+  __shared__ SC xs[cholWavesLdsBytes<TP, SC, G>() / sizeof(SC)];
+  const int w = (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  static_for<0, G>([&](auto Wc) {
+    constexpr int W = Wc;
+    if (w == W) cholSplitTile<TP, SIN, SC, G, W>(B, gM, gU, gD, xs);
   });
 }
 

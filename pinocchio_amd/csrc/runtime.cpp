@@ -1331,10 +1331,10 @@ void cfdCall(rbd_ctx* ctx, const rbd_model* m, int64_t B, const void* q, int64_t
   const TopoOps& o = *m->ops;
   const CView<S> cq{dq, vq.rs, vq.bs}, cv{dv, vv.rs, vv.bs};
   if constexpr (f32) {
-    o.crba_f32(ctx->stream, m->gen.get(), mc, B, cq, View<S>{wM, B, 1}, 0);
+    o.crba_f32(ctx->stream, m->gen.get(), mc, B, cq, View<S>{wM, B, 1}, kMassPattern);
     o.chol_f32(ctx->stream, m->gen.get(), B, CView<S>{wM, B, 1}, View<double>{wU, B, 1}, View<double>{wD, B, 1});
   } else {
-    o.crba_f64(ctx->stream, m->gen.get(), mc, B, cq, View<S>{wM, B, 1}, 0);
+    o.crba_f64(ctx->stream, m->gen.get(), mc, B, cq, View<S>{wM, B, 1}, kMassPattern);
     o.chol_f64(ctx->stream, m->gen.get(), B, CView<S>{wM, B, 1}, View<double>{wU, B, 1}, View<double>{wD, B, 1});
   }
   // nle = rnea(q, v, 0): the acceleration view repeats one zero (both strides 0)
@@ -1378,10 +1378,10 @@ void impulseCall(rbd_ctx* ctx, const rbd_model* m, int64_t B, const void* q, int
   const TopoOps& o = *m->ops;
   const CView<S> cq{dq, vq.rs, vq.bs};
   if constexpr (f32) {
-    o.crba_f32(ctx->stream, m->gen.get(), mc, B, cq, View<S>{wM, B, 1}, 0);
+    o.crba_f32(ctx->stream, m->gen.get(), mc, B, cq, View<S>{wM, B, 1}, kMassPattern);
     o.chol_f32(ctx->stream, m->gen.get(), B, CView<S>{wM, B, 1}, View<double>{wU, B, 1}, View<double>{wD, B, 1});
   } else {
-    o.crba_f64(ctx->stream, m->gen.get(), mc, B, cq, View<S>{wM, B, 1}, 0);
+    o.crba_f64(ctx->stream, m->gen.get(), mc, B, cq, View<S>{wM, B, 1}, kMassPattern);
     o.chol_f64(ctx->stream, m->gen.get(), B, CView<S>{wM, B, 1}, View<double>{wU, B, 1}, View<double>{wD, B, 1});
   }
   const auto kkt = f32 ? (LaunchKkt<S>)o.kkt_f32 : (LaunchKkt<S>)o.kkt_f64;
@@ -1503,11 +1503,11 @@ void cdCall(rbd_ctx* ctx, const rbd_model* m, int64_t B, const void* q, int64_t 
                      ctx->stream, B, nv, nrows, dtab, dsup, CView<S>{wO, B, 1}, CView<S>{wV, B, 1}, CView<S>{wA, B, 1},
                      CView<S>{wJw, B, 1}, View<S>{wJc, B, 1}, View<S>{wG, B, 1});
   if constexpr (f32) {
-    o.crba_f32(ctx->stream, m->gen.get(), mc, B, cq, View<S>{wM, B, 1}, 0);
+    o.crba_f32(ctx->stream, m->gen.get(), mc, B, cq, View<S>{wM, B, 1}, kMassPattern);
     o.chol_f32(ctx->stream, m->gen.get(), B, CView<S>{wM, B, 1}, View<double>{wU, B, 1}, View<double>{wD, B, 1});
     o.rnea_f32(ctx->stream, m->gen.get(), mc, B, cq, cv, zero, View<S>{wN, B, 1});
   } else {
-    o.crba_f64(ctx->stream, m->gen.get(), mc, B, cq, View<S>{wM, B, 1}, 0);
+    o.crba_f64(ctx->stream, m->gen.get(), mc, B, cq, View<S>{wM, B, 1}, kMassPattern);
     o.chol_f64(ctx->stream, m->gen.get(), B, CView<S>{wM, B, 1}, View<double>{wU, B, 1}, View<double>{wD, B, 1});
     o.rnea_f64(ctx->stream, m->gen.get(), mc, B, cq, cv, zero, View<S>{wN, B, 1});
   }
@@ -1579,10 +1579,10 @@ void constraintMatrixCall(rbd_ctx* ctx, const rbd_model* m, int64_t B, const voi
                      ctx->stream, B, nv, nrows, dtab, dsup, CView<S>{wO, B, 1}, CView<S>{wV, B, 1}, CView<S>{wA, B, 1},
                      CView<S>{wJw, B, 1}, View<S>{wJc, B, 1}, View<S>{wGm, B, 1});
   if constexpr (f32) {
-    o.crba_f32(ctx->stream, m->gen.get(), mc, B, cq, View<S>{wM, B, 1}, 0);
+    o.crba_f32(ctx->stream, m->gen.get(), mc, B, cq, View<S>{wM, B, 1}, kMassPattern);
     o.chol_f32(ctx->stream, m->gen.get(), B, CView<S>{wM, B, 1}, View<double>{wU, B, 1}, View<double>{wD, B, 1});
   } else {
-    o.crba_f64(ctx->stream, m->gen.get(), mc, B, cq, View<S>{wM, B, 1}, 0);
+    o.crba_f64(ctx->stream, m->gen.get(), mc, B, cq, View<S>{wM, B, 1}, kMassPattern);
     o.chol_f64(ctx->stream, m->gen.get(), B, CView<S>{wM, B, 1}, View<double>{wU, B, 1}, View<double>{wD, B, 1});
   }
   const auto kkt = f32 ? (LaunchKkt<S>)o.kkt_f32 : (LaunchKkt<S>)o.kkt_f64;

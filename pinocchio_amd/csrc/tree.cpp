@@ -219,20 +219,20 @@ const TProg* prog(GM m) { return m->tree ? m->tree->g.get() : nullptr; }
 // 20586 / 1806).  Matrices of a few hundred bytes stay where they were, but for the
 // derivatives: one configuration is a few cache lines and the serial walk is short (6
 // dofs: equal up to 16,384, FP64 21 / 28 there; derivatives 64 / 58).
-// Batch-fastest output: as long as the lane-per-configuration kernel has less than about
-// one wave per SIMD to hide its serial walk (36 dofs CRBA 53 / 33 at 4,096, 53 / 46 at 8,192,
-// 53 / 67 at 16,384; FP64 58 / 50 at 4,096, 58 / 82 at 8,192; Minv 105 / 50 at 4,096, 110 /
-// 81 at 8,192, 124 / 143 at 16,384; 18 dofs 44 / 33, 46 / 37, 47 / 58; derivatives 36 dofs
-// 233 / 143 at 4,096, 239 / 264 at 8,192, FP64 766 / 485 at 8,192, 934 / 1028 at 16,384;
-// 18 dofs 79 / 68, 86 / 99, FP64 216 / 151, 242 / 246).  FP64 Minv was one solve launch per
-// column: 1627 / 287 at 16,384.
+// Batch-fastest output: where the lane-per-configuration kernels' walk is longer than the
+// phases of the tiles of a CU (36 dofs, CRBA 34 / 24 at one configuration, 34 / 33 at 4,096,
+// 34 / 45 at 8,192, FP64 38 / 31 at 1,024, 38 / 50 at 4,096; 18 dofs 22 / 22 at 1,024; Minv 75 /
+// 52 at 4,096, 79 / 84 at 8,192; 18 dofs 35 / 32, 36 / 35, 37 / 54 at 16,384; derivatives 36
+// dofs 223 / 143 at 4,096, 229 / 264 at 8,192, FP64 766 / 485 at 8,192, 934 / 1028 at 16,384; 18
+// dofs 79 / 68, 86 / 99, FP64 216 / 151, 242 / 246).  FP64 Minv was one solve launch per
+// column: 1599 / 293 at 16,384.
 bool treePays(TreeOp op, bool prebuilt, bool rows, int nv, int es, int64_t B) {
   if (!prebuilt) return true;
   if (op == TreeOp::kDeriv) return rows || B * 4 <= (nv < 12 ? 2048 : 5120) * es;
   if (op == TreeOp::kMinv && es == 8) return true;
   if (rows) return nv * nv * es > 512;
   if (nv < 12) return false;
-  return op == TreeOp::kCrba ? B * es <= 32768 : B <= 10240;
+  return op == TreeOp::kCrba ? B * es <= 12288 : B <= 6144;
 }
 
 // The tree-parallel sweeps take a few phases per level with most lanes idle, so they win
