@@ -44,8 +44,26 @@ def lib():
         L.rbd_version.restype = ctypes.c_char_p
         L.rbd_ctx_stream.restype = ctypes.c_void_p
         L.rbd_ctx_stream.argtypes = [ctypes.c_void_p]
+        # the entry points of the smallest calls take plain integers (pointers and sizes):
+        # declared, ctypes converts them in C instead of through a Python object each
+        for name, sig in _SIGNATURES.items():
+            getattr(L, name).argtypes = [_CTYPES[c] for c in sig]
         _lib = L
     return _lib
+
+
+# p: pointer, l: int64, i: int, u: uint32 flags
+_CTYPES = {"p": ctypes.c_void_p, "l": ctypes.c_int64, "i": ctypes.c_int, "u": ctypes.c_uint32}
+_SIGNATURES = {
+    "rbd_rnea": "ppli" + "pl" * 4 + "u",
+    "rbd_aba": "ppli" + "pl" * 4 + "u",
+    "rbd_crba": "ppli" + "pl" * 2 + "u",
+    "rbd_compute_minverse": "ppli" + "pl" * 2 + "u",
+    "rbd_cholesky_decompose": "ppli" + "pl" * 3 + "u",
+    "rbd_aba_derivatives": "ppli" + "pl" * 3 + "pppl" + "pl" + "u",
+    "rbd_forward_kinematics": "ppli" + "pl" * 4 + "ppl" + "u",
+    "rbd_joint_jacobians": "ppli" + "pl" * 2 + "u",
+}
 
 
 def _check(rc: int):
@@ -173,13 +191,17 @@ class Model:
 # ------------------------------------------------------------------------------------
 # Device-resident engine over torch tensors
 # ------------------------------------------------------------------------------------
+_DTYPES = {}
+
+
 def _dtype_code(t):
-    import torch
-    if t.dtype == torch.float32:
-        return RBD_F32
-    if t.dtype == torch.float64:
-        return RBD_F64
-    raise TypeError(f"unsupported dtype {t.dtype}")
+    if not _DTYPES:
+        import torch
+        _DTYPES.update({torch.float32: RBD_F32, torch.float64: RBD_F64})
+    code = _DTYPES.get(t.dtype)
+    if code is None:
+        raise TypeError(f"unsupported dtype {t.dtype}")
+    return code
 
 
 def _ptr(t):
@@ -208,19 +230,20 @@ class Engine:
 
     def _vec(self, t, rows, name):
         # a dimension of extent 1 may carry any stride
-        if self.layout == "col":
-            ok = t.dim() == 2 and t.shape[1] == rows and (t.stride(1) == 1 or rows == 1)
-            assert ok, f"{name}: expected (B, {rows}) rows-contiguous"
-            return t.shape[0], (t.stride(0) if t.shape[0] > 1 else rows)
-        ok = t.dim() == 2 and t.shape[0] == rows and (t.stride(1) == 1 or t.shape[1] == 1)
-        assert ok, f"{name}: expected ({rows}, B) contiguous"
-        return t.shape[1], (t.stride(0) if rows > 1 else max(t.shape[1], 1))
+        shape = t.shape
+        if len(shape) == 2:
+            n0, n1 = shape
+            s0, s1 = t.stride()
+            if self.layout == "col":
+                if n1 == rows and (s1 == 1 or rows == 1):
+                    return n0, (s0 if n0 > 1 else rows)
+            elif n0 == rows and (s1 == 1 or n1 == 1):
+                return n1, (s0 if rows > 1 else max(n1, 1))
+        what = f"(B, {rows}) rows-contiguous" if self.layout == "col" else f"({rows}, B) contiguous"
+        raise AssertionError(f"{name}: expected {what}")
 
     def _new_vec(self, like, rows, B):
-        import torch
-        if self.layout == "col":
-            return torch.empty((B, rows), dtype=like.dtype, device=like.device)
-        return torch.empty((rows, B), dtype=like.dtype, device=like.device)
+        return like.new_empty((B, rows) if self.layout == "col" else (rows, B))
 
     def _new_mat(self, like, B, dtype=None, zero=False):
         # every kernel writes every entry of its matrices (structural zeros included),
@@ -245,8 +268,8 @@ class Engine:
         _, lda = self._vec(a, m.nv, "a")
         out = self._new_vec(q, m.nv, B) if out is None else out
         _, ldo = self._vec(out, m.nv, "tau")
-        _check(lib().rbd_rnea(m.ctx.handle, m.handle, _i64(B), _dtype_code(q), _ptr(q), _i64(ldq), _ptr(v), _i64(ldv),
-                              _ptr(a), _i64(lda), _ptr(out), _i64(ldo), ctypes.c_uint32(self._flags(async_))))
+        _check(lib().rbd_rnea(m.ctx.handle, m.handle, B, _dtype_code(q), q.data_ptr(), ldq, v.data_ptr(), ldv,
+                              a.data_ptr(), lda, out.data_ptr(), ldo, self._flags(async_)))
         return out
 
     def aba(self, q, v, tau, out=None, async_=False):
@@ -256,8 +279,8 @@ class Engine:
         _, ldt = self._vec(tau, m.nv, "tau")
         out = self._new_vec(q, m.nv, B) if out is None else out
         _, ldo = self._vec(out, m.nv, "ddq")
-        _check(lib().rbd_aba(m.ctx.handle, m.handle, _i64(B), _dtype_code(q), _ptr(q), _i64(ldq), _ptr(v), _i64(ldv),
-                             _ptr(tau), _i64(ldt), _ptr(out), _i64(ldo), ctypes.c_uint32(self._flags(async_))))
+        _check(lib().rbd_aba(m.ctx.handle, m.handle, B, _dtype_code(q), q.data_ptr(), ldq, v.data_ptr(), ldv,
+                             tau.data_ptr(), ldt, out.data_ptr(), ldo, self._flags(async_)))
         return out
 
     def nonlinear_effects(self, q, v, out=None, async_=False):
@@ -332,8 +355,7 @@ class Engine:
         out = self._new_mat(q, B, zero=upper_only) if out is None else out
         ldm = self._mat_arg(out, B, "M")
         flags = self._flags(async_) | (RBD_UPPER_ONLY if upper_only else 0)
-        _check(lib().rbd_crba(m.ctx.handle, m.handle, _i64(B), _dtype_code(q), _ptr(q), _i64(ldq), _ptr(out), _i64(ldm),
-                              ctypes.c_uint32(flags)))
+        _check(lib().rbd_crba(m.ctx.handle, m.handle, B, _dtype_code(q), q.data_ptr(), ldq, out.data_ptr(), ldm, flags))
         return out
 
     def cholesky_decompose(self, M, async_=False):
@@ -405,9 +427,9 @@ class Engine:
         ldo = self._mat_arg(outs[0], B, "out")
         ddq = self._new_vec(q, m.nv, B) if ddq_out is None else ddq_out
         _, ldd = self._vec(ddq, m.nv, "ddq")
-        _check(lib().rbd_aba_derivatives(m.ctx.handle, m.handle, _i64(B), _dtype_code(q), _ptr(q), _i64(ldq), _ptr(v),
-                                         _i64(ldv), _ptr(tau), _i64(ldt), *[_ptr(o) for o in outs], _i64(ldo),
-                                         _ptr(ddq), _i64(ldd), ctypes.c_uint32(self._flags(async_))))
+        _check(lib().rbd_aba_derivatives(m.ctx.handle, m.handle, B, _dtype_code(q), q.data_ptr(), ldq, v.data_ptr(),
+                                         ldv, tau.data_ptr(), ldt, outs[0].data_ptr(), outs[1].data_ptr(),
+                                         outs[2].data_ptr(), ldo, ddq.data_ptr(), ldd, self._flags(async_)))
         return outs[0], outs[1], outs[2], ddq
 
     def forward_kinematics(self, q, v=None, a=None, async_=False):
@@ -424,12 +446,11 @@ class Engine:
         ldv = self._vec(v, m.nv, "v")[1] if v is not None else 0
         lda = self._vec(a, m.nv, "a")[1] if a is not None else 0
         ldva = self._vec(vo, 6 * (nj - 1), "v out")[1] if vo is not None else 0
-        _check(lib().rbd_forward_kinematics(m.ctx.handle, m.handle, _i64(B), _dtype_code(q), _ptr(q), _i64(ldq),
-                                            _ptr(v) if v is not None else None, _i64(ldv),
-                                            _ptr(a) if ao is not None else None, _i64(lda), _ptr(oM), _i64(ldo),
-                                            _ptr(vo) if vo is not None else None,
-                                            _ptr(ao) if ao is not None else None, _i64(ldva),
-                                            ctypes.c_uint32(self._flags(async_))))
+        _check(lib().rbd_forward_kinematics(m.ctx.handle, m.handle, B, _dtype_code(q), q.data_ptr(), ldq,
+                                            v.data_ptr() if v is not None else None, ldv,
+                                            a.data_ptr() if ao is not None else None, lda, oM.data_ptr(), ldo,
+                                            vo.data_ptr() if vo is not None else None,
+                                            ao.data_ptr() if ao is not None else None, ldva, self._flags(async_)))
         return oM, vo, ao
 
     def joint_jacobians(self, q, async_=False):
@@ -438,8 +459,8 @@ class Engine:
         B, ldq = self._vec(q, m.nq, "q")
         J = self._new_vec(q, 6 * m.nv, B)
         _, ldj = self._vec(J, 6 * m.nv, "J")
-        _check(lib().rbd_joint_jacobians(m.ctx.handle, m.handle, _i64(B), _dtype_code(q), _ptr(q), _i64(ldq), _ptr(J),
-                                         _i64(ldj), ctypes.c_uint32(self._flags(async_))))
+        _check(lib().rbd_joint_jacobians(m.ctx.handle, m.handle, B, _dtype_code(q), q.data_ptr(), ldq, J.data_ptr(),
+                                         ldj, self._flags(async_)))
         return J
 
     def joint_jacobians_time_variation(self, q, v, jacobians=True):
@@ -529,8 +550,8 @@ class Engine:
         B, ldq = self._vec(q, m.nq, "q")
         out = self._new_mat(q, B) if out is None else out
         ldm = self._mat_arg(out, B, "Minv")
-        _check(lib().rbd_compute_minverse(m.ctx.handle, m.handle, _i64(B), _dtype_code(q), _ptr(q), _i64(ldq),
-                                          _ptr(out), _i64(ldm), ctypes.c_uint32(self._flags(async_))))
+        _check(lib().rbd_compute_minverse(m.ctx.handle, m.handle, B, _dtype_code(q), q.data_ptr(), ldq, out.data_ptr(),
+                                          ldm, self._flags(async_)))
         return out
 
     def constrained_forward_dynamics(self, q, v, tau, J, gamma, inv_damping=0.0, out=None, lambda_out=None,
