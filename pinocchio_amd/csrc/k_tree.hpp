@@ -42,7 +42,7 @@ struct TProg {
   int oFSeg, nslev;       // its segments (first dof, length) and their levels
   int oPairs;             // (r | c << 8) of the entries with r <= c; read from memory
   int oSeg, nseg;         // chain segments: first dof and length (up to four consecutive dofs)
-  int oCommon;            // bytes, nv x nv: number of common strict ancestors of r and c
+  int oCommon;            // bytes, nv x nv: number of common strict ancestors of r and c; from memory
   int nj, nq, nv, nlev, nlog, nnz;
   uint32_t nvMagic;       // ceil(2^32 / nv): e / nv by multiplication for e < 2^16
 };
@@ -237,17 +237,24 @@ __device__ __forceinline__ void treeMass(const TProg& g, const int16_t* tb, cons
   }
   __syncthreads();
 }
-// scalars of LDS that treeMass needs beside sM
-inline size_t treeMassState(const TProg& g) {
-  return (size_t)g.nj * (kTreeMassJnt * kTreeT + kTreeMassC) + (size_t)g.nv * kTreeMassDof * kTreeT +
-         (size_t)g.nq * kTreeT;
+// scalars of LDS that treeMass needs for its records
+__host__ __device__ inline size_t treeMassState(const TProg& g) {
+  return (size_t)g.nj * kTreeMassJnt * kTreeT + (size_t)g.nv * kTreeMassDof * kTreeT;
+}
+// scalars of the space that holds the constants and q first and M (and what the caller
+// keeps behind it) later: they are dead before the first entry of M is written.  With the
+// pairs' ancestor counts read from memory, not staged, this is a workgroup more per CU
+// (CRBA twice and M^-1 of 10,007 humanoid configurations, FP32: 149 -> 129 us)
+inline size_t treeMassSpace(const TProg& g, size_t later) {
+  const size_t first = (size_t)g.nj * kTreeMassC + (size_t)g.nq * kTreeT;
+  return first > later ? first : later;
 }
 template<class S>
 __device__ __forceinline__ void treeMassTile(const TProg& g, int16_t* tb, int nTab, const S* __restrict__ mc,
                                              CView<S> gq, int64_t b0, int nb, S* state, S* sM) {
   S* sj = state;
   S* sd = sj + g.nj * kTreeMassJnt * kTreeT;
-  S* sc = sd + g.nv * kTreeMassDof * kTreeT;
+  S* sc = sM;
   S* sq = sc + g.nj * kTreeMassC;
   treeStageTab(g, tb, nTab);
   treeStageConsts<S, MC_R, 12, kTreeMassC, 0>(mc, g.nj, sc);
@@ -289,7 +296,8 @@ __device__ __forceinline__ void treePut(View<S> g, int e, const TreeRow<S>& x, i
 
 // CRBA
 template<class S> size_t treeCrbaLds(const TProg& g) {
-  return (size_t)((g.nTab + 7) & ~7) * 2 + (treeMassState(g) + (size_t)(g.nnz + g.nv) * kTreeT) * sizeof(S);
+  return (size_t)((g.nTab + 7) & ~7) * 2 +
+         (treeMassState(g) + treeMassSpace(g, (size_t)(g.nnz + g.nv) * kTreeT)) * sizeof(S);
 }
 template<class S>
 __global__ __launch_bounds__(kTreeMaxThreads) void t_crba(TProg g, const S* __restrict__ mc, int64_t B, CView<S> gq,
@@ -299,8 +307,9 @@ __global__ __launch_bounds__(kTreeMaxThreads) void t_crba(TProg g, const S* __re
   if (b0 >= B) return;
   const int nb = (int)(B - b0 < kTreeT ? B - b0 : kTreeT);
   int16_t* tb = reinterpret_cast<int16_t*>(t_lds);
-  S* sM = reinterpret_cast<S*>(tb + ((g.nTab + 7) & ~7));
-  treeMassTile<S>(g, tb, g.nTab, mc, gq, b0, nb, sM + (g.nnz + g.nv) * kTreeT, sM);
+  S* state = reinterpret_cast<S*>(tb + ((g.nTab + 7) & ~7));
+  S* sM = state + treeMassState(g);
+  treeMassTile<S>(g, tb, g.nTab, mc, gq, b0, nb, state, sM);
   const int nv = g.nv;
   for (int e = threadIdx.x; e < nv * nv; e += blockDim.x) {
     const int c = __umulhi(e, g.nvMagic), r = e - c * nv;
@@ -475,13 +484,13 @@ __device__ __forceinline__ void treeFactor(const TProg& g, const int16_t* tb, S*
 template<class S> size_t treeMinvLds(const TProg& g) {
   const size_t state = treeMassState(g), w = (size_t)g.nnz * kTreeT;
   return (size_t)((g.nTabFactor + 7) & ~7) * 2 +
-         ((state > w ? state : w) + (size_t)(g.nnz + 2 * g.nv) * kTreeT) * sizeof(S);
+         ((state > w ? state : w) + treeMassSpace(g, (size_t)(g.nnz + 2 * g.nv) * kTreeT)) * sizeof(S);
 }
 template<class S>
 __device__ __forceinline__ TreeRow<S> treeMinvEntry(const TProg& g, const int16_t* tb, const S* sW, const S* sDi, int e) {
   const int c = __umulhi(e, g.nvMagic), r = e - c * g.nv;
   const int lo = r < c ? r : c, hi = r < c ? c : r;
-  const int n = reinterpret_cast<const uint8_t*>(tb + g.oCommon)[e], cl = tb[g.oCp + lo];
+  const int n = reinterpret_cast<const uint8_t*>(g.tab + g.oCommon)[e], cl = tb[g.oCp + lo];
   TreeRow<S> x{};
 #pragma unroll 2
   for (int k = 0; k < n; ++k) {
@@ -512,9 +521,10 @@ __global__ __launch_bounds__(kTreeMaxThreads) void t_minv(TProg g, const S* __re
   if (b0 >= B) return;
   const int nb = (int)(B - b0 < kTreeT ? B - b0 : kTreeT);
   int16_t* tb = reinterpret_cast<int16_t*>(t_lds);
-  S* sM = reinterpret_cast<S*>(tb + ((g.nTabFactor + 7) & ~7));
+  S* sW = reinterpret_cast<S*>(tb + ((g.nTabFactor + 7) & ~7));
+  const size_t state = treeMassState(g), nW = (size_t)g.nnz * kTreeT;
+  S* sM = sW + (state > nW ? state : nW);
   S* sDi = sM + (g.nnz + g.nv) * kTreeT;
-  S* sW = sDi + g.nv * kTreeT;
   treeMassTile<S>(g, tb, g.nTabFactor, mc, gq, b0, nb, sW, sM);
   treeFactor<S>(g, tb, sM, sDi, sW);
   for (int e = threadIdx.x; e < g.nv * g.nv; e += blockDim.x) treePut(gX, e, treeMinvEntry<S>(g, tb, sW, sDi, e), b0, nb);
@@ -818,14 +828,17 @@ __global__ __launch_bounds__(kTreeMaxThreads) void t_dsolve(TProg g, int64_t B, 
 // articulated inertias up by levels of the tree, a parent adding what its children left in
 // their records.  Records: the joint transform (12), then
 //   RNEA: v, later the force; a, later the force moved to the parent;
-//   ABA: inertia (21) and bias force, later those moved to the parent; v, later the
-//   acceleration; the accumulated bias, later U / D; u / D - bias . U / D.
+//   ABA (of the transform the rotation only: a revolute joint's translation is a constant):
+//   inertia (21) and bias force, later those moved to the parent; v, later the acceleration;
+//   the accumulated bias, later U / D; u / D - bias . U / D.  (With this and the
+//   smaller space of CRBA, the forward dynamics and mass matrix of 16,384 configurations of a
+//   27-dof random tree went from 211 us to 193.)
 // One workgroup's sweep is some 20 phases of short work for its few workers per level: two
 // waves and a small tile leave room for several workgroups per CU.
 // ---------------------------------------------------------------------------------------
 constexpr int kTreeDynThreads = 128;  // a level has few joints; 16 workers
 constexpr int kTreeDynC = 23;         // staged constants: placement, mass, lever, inertia
-constexpr int kTreeRneaJnt = 25, kTreeAbaJnt = 53;
+constexpr int kTreeRneaJnt = 25, kTreeAbaJnt = 49;
 template<class S> size_t treeDynLds(const TProg& g, int rec) {
   return (size_t)((g.nTabDyn + 7) & ~7) * 2 +
          ((size_t)g.nj * (rec * kTreeT + kTreeDynC) + (size_t)(g.nq + 3 * g.nv) * kTreeT) * sizeof(S);
@@ -947,15 +960,19 @@ __global__ __launch_bounds__(kTreeDynThreads) void t_aba(TProg g, const S* __res
   const int b = treeB(), w = treeW(), NW = treeNW();
   const S* __restrict__ arm = mc + g.nj * MC_REC;
   const Mot<S> a0 = mcGravityNeg(arm, g.nv);
-  constexpr int kI = 12, kP = 33, kV = 39, kC = 45, kS = 51;  // inertia, force, v, bias, scalar
+  constexpr int kI = 9, kP = 30, kV = 36, kC = 42, kS = 48;  // inertia, force, v, bias, scalar
   auto jnt = [&](int j) { return TRec<S>{t.sj + j * kTreeAbaJnt * kTreeT + b}; };
+  // a revolute joint's transform (a free flyer's is used once, at its solve)
+  auto jointX = [&](int j) {
+    return Xform<S>{jnt(j).template get<R3<S>>(0), ldsConst<V3<S>>(t.sc + j * kTreeDynC + 9)};
+  };
   for (int j = 1 + w; j < g.nj; j += NW)
-    jnt(j).put(0, treeJointX(t.sc + j * kTreeDynC, tb[j * TJ_REC + TJ_TYPE], t.sq + b, tb[j * TJ_REC + TJ_IQ]));
+    jnt(j).put(0, treeJointX(t.sc + j * kTreeDynC, tb[j * TJ_REC + TJ_TYPE], t.sq + b, tb[j * TJ_REC + TJ_IQ]).R);
   for (int l = 0; l < g.nlev; ++l) {
     __syncthreads();
     for (int e = tb[g.oJLvl + l] + w, e1 = tb[g.oJLvl + l + 1]; e < e1; e += NW) {
       const int j = tb[g.oJList + e], p = tb[j * TJ_REC + TJ_PARENT], ty = tb[j * TJ_REC + TJ_TYPE];
-      const Xform<S> X = jnt(j).template get<Xform<S>>(0);
+      const Xform<S> X = jointX(j);
       const Mot<S> vJ = treeJointMot(ty, t.sv + tb[j * TJ_REC + TJ_IV] * kTreeT + b);
       Mot<S> v = vJ;
       if (p > 0) v = v + actInv(X, jnt(p).template get<Mot<S>>(kV));
@@ -984,10 +1001,9 @@ __global__ __launch_bounds__(kTreeDynThreads) void t_aba(TProg g, const S* __res
         symAdd(Ia, jnt(c).template get<Sym6<S>>(kI));
         pA = pA + jnt(c).template get<Frc<S>>(kP);
       }
-      const Xform<S> X = jnt(j).template get<Xform<S>>(0);
       if (ty == JT_FF) {
         // root free flyer: D = Ia + armature (6x6, FP64 LLT), qdd = D^-1 (tau - pA - Ia a')
-        const Mot<S> ap = actInv(X, a0);
+        const Mot<S> ap = actInv(treeJointX(t.sc + j * kTreeDynC, ty, t.sq + b, tb[j * TJ_REC + TJ_IQ]), a0);
         const Frc<S> Iap = symMul6(Ia, ap);
         double A[21], x[6];
 #pragma unroll
@@ -1018,6 +1034,7 @@ __global__ __launch_bounds__(kTreeDynThreads) void t_aba(TProg g, const S* __res
           symRank1Sub(Ia, U, Dinv);
           const Mot<S> ci = crossMM(jnt(j).template get<Mot<S>>(kV), axisMot(ax, t.sv[iv * kTreeT + b]));
           const Frc<S> pa = pA + symMul6(Ia, ci) + scale(Dinv * u, U);
+          const Xform<S> X = jointX(j);
           jnt(j).put(kI, transportUp(X, Ia));
           jnt(j).put(kP, act(X, pa));
         }
@@ -1029,7 +1046,7 @@ __global__ __launch_bounds__(kTreeDynThreads) void t_aba(TProg g, const S* __res
     for (int e = tb[g.oJLvl + l] + w, e1 = tb[g.oJLvl + l + 1]; e < e1; e += NW) {
       const int j = tb[g.oJList + e], p = tb[j * TJ_REC + TJ_PARENT], ty = tb[j * TJ_REC + TJ_TYPE];
       if (ty == JT_FF) continue;
-      const Mot<S> x = actInv(jnt(j).template get<Xform<S>>(0), p > 0 ? jnt(p).template get<Mot<S>>(kV) : a0);
+      const Mot<S> x = actInv(jointX(j), p > 0 ? jnt(p).template get<Mot<S>>(kV) : a0);
       const S qdd = t.sj[(j * kTreeAbaJnt + kS) * kTreeT + b] - dot(x, jnt(j).template get<Frc<S>>(kC));
       t.so[tb[j * TJ_REC + TJ_IV] * kTreeT + b] = qdd;
       jnt(j).put(kV, x + axisMot(ty - JT_RX, qdd));

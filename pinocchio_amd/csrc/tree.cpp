@@ -161,9 +161,9 @@ TreeProgram* buildTreeProgram(int nj, const int* parents, const int* types, std:
       while (k < anc[r].size() && k < anc[c].size() && anc[r][k] == anc[c][k]) ++k;
       com[(size_t)c * nv + r] = (uint8_t)k;
     }
+  g.nTabFactor = (int)tab.size();
   g.oCommon = (int)tab.size();
   for (size_t k = 0; k + 1 < com.size(); k += 2) tab.push_back((int16_t)(com[k] | com[k + 1] << 8));
-  g.nTabFactor = (int)tab.size();
   g.oPairs = (int)tab.size();
   for (int c = 0; c < nv; ++c)
     for (int r = 0; r <= c; ++r) tab.push_back((int16_t)(r | c << 8));
