@@ -193,28 +193,42 @@ void launchAbaDSolve(hipStream_t st, GM, int64_t B, CView<S> U, CView<S> D, View
 }
 
 
-template<class TP, class S, int G>
-void launchKinWaves(hipStream_t st, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> oM,
-                    View<S> vo, View<S> ao, View<S> J, const KinMask& want) {
-  if (kinRows(oM, vo, ao, J))
-    hipLaunchKernelGGL((k_kin<TP, S, true, G>), dim3(gridFor(B)), dim3(kTile * G), 0, st, mc, B, q, v, a, oM, vo, ao,
-                       J, want);
-  else
-    hipLaunchKernelGGL((k_kin<TP, S, false, G>), dim3(gridFor(B)), dim3(kTile * G), 0, st, mc, B, q, v, a, oM, vo, ao,
-                       J, want);
-}
-// Four waves per tile up to one tile per CU, or two when only the Jacobian is written; beyond
-// that the stores bound the kernel and one wave's come in better order (humanoid, us per
-// call, one wave / four: placements and motions 56 / 36 at 16,384, 60 / 69 at 30,011, FP64
-// rows 215 / 256 at 65,536; Jacobian 33 / 24, 34 / 28, rows 45 / 49 at 65,536).
+// Outputs by rows.  Runs of a lane's own row while the tiles leave the chip idle: a tile's
+// latency counts there, and staging the runs adds to it.  Beyond, staged (us per call, own /
+// staged; humanoid, placements and motions: 33 / 35 at 4,096, 36 / 36 at 8,192, 48 / 41 at
+// 16,384, 62 / 50 at 30,011, 123 / 80 at 65,536, FP64 40 / 40, 46 / 43, 54 / 47, 85 / 69,
+// 209 / 194; arm, one wave per tile, 28 / 30 at 16,384, 31 / 31 at 24,000, 47 / 38 at
+// 65,536; Jacobian 25 / 26 at 16,384, 29 / 27 at 24,000, FP64 38 / 43 at 30,011, 65 / 58 at
+// 48,000).
+// Four waves per tile wherever the tree splits; element by element (batch-fastest) up to
+// one tile per CU, or two when only the Jacobian is written: there the stores bound the
+// kernel beyond that, and one wave's come in better order (humanoid, one wave / four:
+// placements and motions 56 / 36 at 16,384, 60 / 69 at 30,011, Jacobian 33 / 24, 34 / 28).
 template<class TP, class S>
 void launchKin(hipStream_t st, GM, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> oM, View<S> vo,
                View<S> ao, View<S> J, const KinMask& want) {
-  if constexpr (treeSplits<TP>()) {
-    if (B <= (int64_t)256 * kTile * (oM.p || vo.p ? 1 : 2))
-      return launchKinWaves<TP, S, 4>(st, mc, B, q, v, a, oM, vo, ao, J, want);
+  constexpr int G = treeSplits<TP>() ? 4 : 1;
+  constexpr int64_t perCu = 256 * kTile;  // configurations of one tile per CU
+  auto launch = [&](auto Oc, auto Gc) {
+    constexpr KinOut O = KinOut(int(Oc));
+    constexpr int g = Gc;
+    hipLaunchKernelGGL((k_kin<TP, S, O, g>), dim3(gridFor(B)), dim3(kTile * g), 0, st, mc, B, q, v, a, oM, vo, ao, J,
+                       want);
+  };
+  const bool onlyJ = !oM.p && !vo.p;
+  if (kinRows(oM, vo, ao, J)) {
+    constexpr int bytes = (kinInScalars<TP>() + kinRunScalars<S, KinOut::kStaged>() * G) * (int)sizeof(S);
+    if constexpr (bytes <= 160 * 1024) {
+      const int64_t own = G == 1 ? perCu * 3 / 2 : !onlyJ ? perCu / 2 : sizeof(S) == 8 ? perCu * 2 : perCu;
+      if (B > own && want.joints == ~0ull && want.columns == ~0ull)
+        return launch(IC<(int)KinOut::kStaged>{}, IC<G>{});
+    }
+    return launch(IC<(int)KinOut::kRuns>{}, IC<G>{});
   }
-  launchKinWaves<TP, S, 1>(st, mc, B, q, v, a, oM, vo, ao, J, want);
+  if constexpr (G > 1) {
+    if (B <= perCu * (onlyJ ? 2 : 1)) return launch(IC<(int)KinOut::kElements>{}, IC<G>{});
+  }
+  launch(IC<(int)KinOut::kElements>{}, IC<1>{});
 }
 
 template<class TP, class S>

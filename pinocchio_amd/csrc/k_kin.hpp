@@ -41,14 +41,67 @@ template<class S> bool kinRows(View<S> M, View<S> V, View<S> A, View<S> J) {
   return ok(M, 16 / sizeof(S)) && ok(V, 2) && ok(A, 2) && ok(J, 2);
 }
 
-// kRows: every output that is present passed kinRows.  G > 1: G waves share the tile, each
-// running the trunk and its subtrees (WaveSplit); nothing goes back up, so there is nothing
-// to hand over.  (Humanoid, 16,384 configurations, placements, motions and Jacobian: 45 us
-// on one wave, the serial walk of one tile per CU.)
-template<class TP, class S, bool kRows, int G, int W>
+// How the outputs leave: element by element (any strides), as runs of a lane's own row, or
+// as runs through LDS (kRunJoints<S> joints at a time: the wave's lanes write the runs of
+// consecutive joints next to each other, so that neighbouring lanes store neighbouring
+// vectors of one configuration).  A lane's own runs are a request of the L2 per 8 or 16
+// bytes, which bounds the kernel once the tiles fill the chip at any number of waves.
+enum class KinOut { kElements, kRuns, kStaged };
+template<class S> constexpr int kRunJoints = sizeof(S) == 4 ? 3 : 2;
+// Joints whose outputs wave W stores, in groups of consecutive indices: size[i] is the
+// group's if joint i is its last, else 0.
+template<class TP, int G, int W, int N> struct KinRuns {
+  int size[TP::NJ] = {};
+  constexpr KinRuns() {
+    constexpr auto& T = TP::T;
+    constexpr WaveSplit<TP, G> WS{};
+    int n = 0, last = -1;
+    for (int k = 0; k < TP::NJ - 1; ++k) {
+      const int i = T.order[k];
+      if (!WS.runs(i, W) || WS.writer(i) != W) continue;
+      if (n > 0 && (i != last + 1 || n == N)) {
+        size[last] = n;
+        n = 0;
+      }
+      ++n;
+      last = i;
+    }
+    if (n > 0) size[last] = n;
+  }
+};
+// pitch of a configuration's space: whole 16-byte vectors, an odd number of them
+template<class S> constexpr int kRunPitch() {
+  constexpr int V = 16 / (int)sizeof(S), n = 12 * kRunJoints<S>;
+  return n / V % 2 ? n : n + V;
+}
+// N scalars of each of the wave's configurations from LDS to dst + c bs
+template<int N, int V, class S>
+__device__ __forceinline__ void flushRuns(const S* st, S* dst, int64_t bs, int nb) {
+  typedef S Vec __attribute__((ext_vector_type(V)));
+  constexpr int nv = N / V;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+  for (int k = 0; k < nv; ++k) {
+    const int it = k * kTile + laneId(), c = it / nv, u = it - c * nv;
+    if (c < nb)
+      *reinterpret_cast<Vec*>(dst + c * bs + u * V) = *reinterpret_cast<const Vec*>(st + c * kRunPitch<S>() + u * V);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+// scalars of LDS: the inputs, each wave's space of KinOut::kStaged
+template<class TP> constexpr int kinInScalars() { return (kinLdsRows<TP>() * kPitch + 3) / 4 * 4; }
+template<class S, KinOut O> constexpr int kinRunScalars() { return O == KinOut::kStaged ? kTile * kRunPitch<S>() : 0; }
+
+// KinOut::kRuns, kStaged: every output that is present passed kinRows; kStaged: all joints
+// are wanted.  G > 1: G waves share the tile, each running the trunk and its subtrees
+// (WaveSplit); nothing goes back up, so there is nothing to hand over.  (Humanoid, 16,384
+// configurations, placements, motions and Jacobian: 45 us on one wave, the serial walk of
+// one tile per CU; 14 on four.)
+template<class TP, class S, KinOut O, int G, int W>
 __device__ __forceinline__ void kinTile(const S* __restrict__ mc_in, int64_t B, CView<S> gq, CView<S> gv, CView<S> ga,
                                         View<S> gM, View<S> gV, View<S> gA, View<S> gJ, KinMask want,
-                                        S* __restrict__ lds) {
+                                        S* __restrict__ lds, S* __restrict__ runs) {
   constexpr auto& T = TP::T;
   constexpr int NJ = TP::NJ, NQ = T.nq, NV = T.nv;
   constexpr WaveSplit<TP, G> WS{};
@@ -70,23 +123,26 @@ __device__ __forceinline__ void kinTile(const S* __restrict__ mc_in, int64_t B, 
 
   Xform<S> oM[NJ];
   Mot<S> vj[NJ], aj[NJ];
-  // N consecutive rows of an output; kRows: one run of the configuration's memory
+  constexpr bool kStaged = O == KinOut::kStaged;
+  // N consecutive rows of an output; kRuns: one run of the configuration's memory
   auto put = [&](auto Nc, View<S> g, int row, const S* x) {
     constexpr int N = Nc;
     if (!live) return;
-    if constexpr (kRows) {
+    if constexpr (O == KinOut::kRuns) {
       putRun<N>(g.p + b * g.bs + row, x);
     } else {
 #pragma unroll
       for (int k = 0; k < N; ++k) stOut(&g.p[(int64_t)(row + k) * g.rs + b * g.bs], x[k]);
     }
   };
+  constexpr KinRuns<TP, G, W, kRunJoints<S>> KR{};
+  S* run = runs + L * kRunPitch<S>();
 
   static_for<0, NJ - 1>([&](auto K) {
     constexpr int i = TP::T.order[K];
     if constexpr (WS.runs(i, W)) {
     constexpr bool mine = WS.writer(i) == W;
-    const bool out = mine && ((want.joints >> i) & 1);
+    const bool out = !kStaged && mine && ((want.joints >> i) & 1);
     stepFence();
     const S* __restrict__ mc = stepConsts(mc_in);
     constexpr int p = TP::T.parent[i];
@@ -136,7 +192,7 @@ __device__ __forceinline__ void kinTile(const S* __restrict__ mc_in, int64_t B, 
         if (out) put(IC<6>{}, gA, (i - 1) * 6, oa);
       }
     }
-    if (mine && gJ.p && ((want.columns >> i) & 1)) {
+    if (!kStaged && mine && gJ.p && ((want.columns >> i) & 1)) {
 #pragma unroll
       for (int k = 0; k < nvi; ++k) {
         const Mot<S> c = worldAxis<ty>(oM[i], k);
@@ -144,19 +200,57 @@ __device__ __forceinline__ void kinTile(const S* __restrict__ mc_in, int64_t B, 
         put(IC<6>{}, gJ, (iv + k) * 6, o);
       }
     }
+    if constexpr (kStaged && KR.size[i] > 0) {
+      constexpr int n = KR.size[i], i0 = i - n + 1;  // the group
+      constexpr int d0 = TP::T.iv[i0], nd = iv + nvi - d0;
+      if (gM.p) {
+        static_for<0, n>([&](auto Jc) {
+          constexpr int j = i0 + Jc;
+          const R3<S>& R = oM[j].R;
+          const S r12[12] = {R.m00, R.m01, R.m02, R.m10, R.m11, R.m12, R.m20, R.m21, R.m22,
+                             oM[j].p.x, oM[j].p.y, oM[j].p.z};
+          putRun<12>(run + (j - i0) * 12, r12);
+        });
+        flushRuns<12 * n, 16 / sizeof(S)>(runs, gM.p + b0 * gM.bs + (i0 - 1) * 12, gM.bs, nb);
+      }
+      auto motions = [&](View<S> g, const Mot<S>* m) {
+        static_for<0, n>([&](auto Jc) {
+          constexpr int j = i0 + Jc;
+          const S o[6] = {m[j].l.x, m[j].l.y, m[j].l.z, m[j].a.x, m[j].a.y, m[j].a.z};
+          putRun<6>(run + (j - i0) * 6, o);
+        });
+        flushRuns<6 * n, 2>(runs, g.p + b0 * g.bs + (i0 - 1) * 6, g.bs, nb);
+      };
+      if (wantV) motions(gV, vj);
+      if (wantA) motions(gA, aj);
+      if (gJ.p) {  // a free flyer's columns may take two turns
+        constexpr int most = 2 * kRunJoints<S>;
+        static_for<0, (nd + most - 1) / most>([&](auto Qc) {
+          constexpr int c0 = d0 + Qc * most, nc = d0 + nd - c0 < most ? d0 + nd - c0 : most;
+          static_for<0, nc>([&](auto Cc) {
+            constexpr int c = c0 + Cc, j = TP::T.dofJoint[c];
+            const Mot<S> m = worldAxis<TP::T.type[j]>(oM[j], c - TP::T.iv[j]);
+            const S o[6] = {m.l.x, m.l.y, m.l.z, m.a.x, m.a.y, m.a.z};
+            putRun<6>(run + Cc * 6, o);
+          });
+          flushRuns<6 * nc, 2>(runs, gJ.p + b0 * gJ.bs + c0 * 6, gJ.bs, nb);
+        });
+      }
+    }
     }
   });
 }
-template<class TP, class S, bool kRows, int G>
+template<class TP, class S, KinOut O, int G>
 __global__ __launch_bounds__(64 * G) void k_kin(const S* __restrict__ mc, int64_t B, CView<S> gq, CView<S> gv,
                                                 CView<S> ga, View<S> gM, View<S> gV, View<S> gA, View<S> gJ,
                                                 KinMask want) {
   static_assert(TP::NJ <= 64, "one mask bit per joint");
-  __shared__ S lds[kinLdsRows<TP>() * kPitch];
+  constexpr int nIn = kinInScalars<TP>(), nRun = kinRunScalars<S, O>();
+  __shared__ __align__(16) S lds[nIn + nRun * G];
   const int w = G > 1 ? (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
   static_for<0, G>([&](auto Wc) {
     constexpr int W = Wc;
-    if (w == W) kinTile<TP, S, kRows, G, W>(mc, B, gq, gv, ga, gM, gV, gA, gJ, want, lds);
+    if (w == W) kinTile<TP, S, O, G, W>(mc, B, gq, gv, ga, gM, gV, gA, gJ, want, lds, lds + nIn + nRun * W);
   });
 }
 

@@ -187,3 +187,30 @@ def test_kinematics_rows(ctx, dt, bar, pad):
             x = out[k].double().cpu().numpy()
             assert rel_err_cols(x[:, :n].T, ref[k].T).max() < bar, (d.name, k, pad)
             assert (x[:, n:] == 7.0).all()
+
+
+@pytest.mark.parametrize("dt,bar", [(torch.float32, 2e-6), (torch.float64, 1e-13)])
+def test_kinematics_rows_staged(ctx, dt, bar):
+    """The batch sizes whose row outputs go through LDS, with a last tile of one
+    configuration and gaps between the rows; against the batch-fastest outputs (the same sums
+    per configuration: the bar of the test above)."""
+    for d, B in ((M.arm7(), 32769), (M.random60(), 32769), (M.humanoid36(), 32769), (M.quadruped18(), 8193)):
+        m = pa.Model(ctx, d)
+        q, v, a = (_dev(x, "col", dt) for x in _inputs(d, B, dt)[:3])
+        eb = pa.Engine(m, "batch")
+        ref = [*eb.forward_kinematics(*(x.t().contiguous() for x in (q, v, a))), eb.joint_jacobians(q.t().contiguous())]
+        code = pa.RBD_F32 if dt == torch.float32 else pa.RBD_F64
+        p, i = pa._ptr, pa._i64
+        out = [torch.full((B, r.numel() // B + pad), 7.0, dtype=dt, device="cuda") for r, pad in zip(ref, (4, 2, 2, 6))]
+        ld = [i(x.stride(0)) for x in out]
+        pa._check(pa.lib().rbd_forward_kinematics(
+            ctx.handle, m.handle, i(B), code, p(q), i(d.nq), p(v), i(d.nv), p(a), i(d.nv), p(out[0]), ld[0],
+            p(out[1]), p(out[2]), ld[1], ctypes.c_uint32(0)))
+        pa._check(pa.lib().rbd_joint_jacobians(ctx.handle, m.handle, i(B), code, p(q), i(d.nq), p(out[3]), ld[3],
+                                               ctypes.c_uint32(0)))
+        for x, r in zip(out, ref):
+            r = r.reshape(-1, B).t()
+            n = r.shape[1]
+            assert ((x[:, :n] - r).abs().amax(1) <= bar * r.abs().amax(1)).all(), d.name
+            assert (x[:, n:] == 7.0).all()
+
