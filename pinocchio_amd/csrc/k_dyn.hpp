@@ -43,7 +43,7 @@ template<class TP> constexpr int dynLdsRows() { return TP::T.nq + 2 * TP::T.nv; 
 // G > 1: G waves share the tile and split the tree by subtrees (WaveSplit, as in ABA); this
 // is the body of wave W.  A subtree hands its force (6 scalars) to its trunk parent through
 // an LDS slot (xs); the trunk's tau stays in registers until every wave has read its a.
-// (Humanoid, 50,021 rows: 34.6 us with one wave, the serial walk of one tile per SIMD; 24
+// (Humanoid, 50,021 rows: 34.6 us with one wave, the serial walk of one tile per SIMD; 25
 // with four, 37 KB and four workgroups per CU.)
 constexpr int kRneaSlot = 6;
 template<class TP, class S, int kU = kStageU, int G = 1, int W = 0>

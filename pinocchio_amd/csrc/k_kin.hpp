@@ -7,7 +7,7 @@
 //   v_i = vJ + liMi^-1 v_parent                              -> gV (6 per joint, local frame)
 //   a_i = S qdd + v_i x vJ + liMi^-1 a_parent                -> gA (6 per joint, local frame)
 //   J[:, dof] = oMi.act(S_dof)  (WORLD frame)                -> gJ (element r + 6 dof)
-// Any output may be absent (null pointer); all outputs leave with nontemporal stores.
+// Any output may be absent (null pointer).
 #pragma once
 
 #include "k_crba.hpp"
@@ -20,8 +20,9 @@ template<class TP> constexpr int kinLdsRows() { return TP::T.nq + 2 * TP::T.nv; 
 // N consecutive scalars in vectors of 16 (placements) or two scalars (motions, columns):
 // with one configuration per row a lane's outputs are runs in its own row, a lane apart by
 // the row length.  Ordinary stores, so that the L2 completes a line from the runs of
-// neighbouring joints: one nontemporal scalar at a time took 952 us where this takes 43
-// (humanoid, 30,011 rows, 112 MB; 2.6 TB/s).
+// neighbouring joints: one nontemporal scalar at a time took 952 us where this took 43
+// (humanoid, placements and motions of 30,011 rows, 86 MB; staged on four waves, below, 31:
+// 2.8 TB/s).
 template<int N, class S> __device__ __forceinline__ void putRun(S* dst, const S* x) {
   constexpr int V = N == 12 ? 16 / (int)sizeof(S) : 2;
   typedef S Vec __attribute__((ext_vector_type(V)));

@@ -244,7 +244,7 @@ __host__ __device__ inline size_t treeMassState(const TProg& g) {
 // scalars of the space that holds the constants and q first and M (and what the caller
 // keeps behind it) later: they are dead before the first entry of M is written.  With the
 // pairs' ancestor counts read from memory, not staged, this is a workgroup more per CU
-// (CRBA twice and M^-1 of 10,007 humanoid configurations, FP32: 149 -> 129 us)
+// (CRBA and M^-1 of 10,007 humanoid configurations, FP32: 149 -> 129 us)
 inline size_t treeMassSpace(const TProg& g, size_t later) {
   const size_t first = (size_t)g.nj * kTreeMassC + (size_t)g.nq * kTreeT;
   return first > later ? first : later;
@@ -335,7 +335,7 @@ __global__ __launch_bounds__(kTreeMaxThreads) void t_crba(TProg g, const S* __re
 // 3 of a level reads nothing that 1 of the next writes: one phase.  With W explicit, M^-1 =
 // W^T D^-1 W is a sum over ancestors without a chain from row to row.  One level per dof
 // instead of per segment (three times the phases, one column per item) took 21 us of a
-// tile, triangular sweeps with U 40 us, against 9.
+// tile, triangular sweeps with U 40 us, against 13 (humanoid, FP32).
 // Leaves 1 / D in sDi and W in sW.
 // ---------------------------------------------------------------------------------------
 struct __align__(8) TItem {
@@ -714,7 +714,7 @@ __global__ __launch_bounds__(kTreeMaxThreads) void t_rnead(TProg g, const S* __r
 // and subtree, which alone are staged and summed over.  A worker takes four rows and a
 // segment of one X: eight LDS reads for sixteen multiply-adds.  (Two sparse products with W
 // are half the multiply-adds, but two phases of short sums each: 45 us of a tile against
-// 15.)  R segments per round.
+// 22, humanoid FP32.)  R segments per round.
 // gridDim.y == 3, for batches whose tiles alone leave CUs idle: y = 0, 1 the even and odd
 // rounds, y = 2 M^-1 (each repeats the factor).
 // LDS: M^-1 [row][row][configuration]; the factor, over which the rounds' X goes.
