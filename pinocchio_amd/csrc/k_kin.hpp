@@ -143,7 +143,7 @@ __device__ __forceinline__ void kinTile(const S* __restrict__ mc_in, int64_t B, 
     constexpr int i = TP::T.order[K];
     if constexpr (WS.runs(i, W)) {
     constexpr bool mine = WS.writer(i) == W;
-    const bool out = !kStaged && mine && ((want.joints >> i) & 1);
+    const bool out = !kStaged && mine && (want.joints & KinMask::bit(i));
     stepFence();
     const S* __restrict__ mc = stepConsts(mc_in);
     constexpr int p = TP::T.parent[i];
@@ -193,7 +193,7 @@ __device__ __forceinline__ void kinTile(const S* __restrict__ mc_in, int64_t B, 
         if (out) put(IC<6>{}, gA, (i - 1) * 6, oa);
       }
     }
-    if (!kStaged && mine && gJ.p && ((want.columns >> i) & 1)) {
+    if (!kStaged && mine && gJ.p && (want.columns & KinMask::bit(i))) {
 #pragma unroll
       for (int k = 0; k < nvi; ++k) {
         const Mot<S> c = worldAxis<ty>(oM[i], k);
@@ -245,7 +245,6 @@ template<class TP, class S, KinOut O, int G>
 __global__ __launch_bounds__(64 * G) void k_kin(const S* __restrict__ mc, int64_t B, CView<S> gq, CView<S> gv,
                                                 CView<S> ga, View<S> gM, View<S> gV, View<S> gA, View<S> gJ,
                                                 KinMask want) {
-  static_assert(TP::NJ <= 64, "one mask bit per joint");
   constexpr int nIn = kinInScalars<TP>(), nRun = kinRunScalars<S, O>();
   __shared__ __align__(16) S lds[nIn + nRun * G];
   const int w = G > 1 ? (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;

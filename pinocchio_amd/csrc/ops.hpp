@@ -37,8 +37,10 @@ using LaunchAbaDSolve = void (*)(hipStream_t, GM, int64_t B, CView<S> U, CView<S
 
 // Joints and dofs whose outputs are wanted (bit i: joint i's placement and motions; the
 // Jacobian columns of joint i's dofs): the constraint rows need those of their joints only.
+// Joints 64 apart share a bit (a tree may have any number): more may be written than asked.
 struct KinMask {
   uint64_t joints = ~0ull, columns = ~0ull;
+  static constexpr uint64_t bit(int joint) { return 1ull << (joint & 63); }
 };
 
 // forward kinematics / joint Jacobians: outputs placements, local velocities and

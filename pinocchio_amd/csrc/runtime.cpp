@@ -1438,8 +1438,8 @@ KinMask constraintMask(const rbd_model* m, int ncon, const rbd_rigid_constraint*
   KinMask k{0, 0};
   for (int c = 0; c < ncon; ++c)
     for (int j : {cons[c].joint1_id, cons[c].joint2_id}) {
-      k.joints |= 1ull << (j & 63);
-      for (int a = j; a > 0; a = m->parents[a]) k.columns |= 1ull << (a & 63);
+      k.joints |= KinMask::bit(j);
+      for (int a = j; a > 0; a = m->parents[a]) k.columns |= KinMask::bit(a);
     }
   return k;
 }

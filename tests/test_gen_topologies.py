@@ -1,7 +1,10 @@
 """The build's topology generator: a user's URDF / MJCF robots join the prebuilt list
-(`make -C pinocchio_amd/csrc ROBOTS=...`).  Generated into a temporary folder; nothing is
-compiled here."""
+(`make -C pinocchio_amd/csrc ROBOTS=...`).  Generated into a temporary folder; one unit's syntax
+is checked with the device compiler."""
+import glob
 import os
+import shutil
+import subprocess
 import sys
 
 import pytest
@@ -49,3 +52,27 @@ def test_user_robots_join_the_list(tmp_path):
         assert f"struct Topo_{name} " in inc
     with pytest.raises(ValueError):
         G.main(str(out), f"{arm}:floating")
+
+
+@pytest.mark.parametrize("family", ["kin", "crba_w4", "chol_w4fd", "dyn_rnea_w4"])
+def test_a_robot_of_70_joints_compiles(tmp_path, family):
+    """More joints than a 64-bit mask has bits (a humanoid with hands): a torso of four joints
+    with branches of six."""
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    links, joints = ["base"], []
+    for k in range(70):
+        parent = links[4] if k >= 4 and (k - 4) % 6 == 0 else links[-1]
+        axis = ("1 0 0", "0 1 0", "0 0 1")[k % 3]
+        links.append(f"l{k}")
+        joints.append(f'<joint name="j{k}" type="revolute"><parent link="{parent}"/><child link="l{k}"/>'
+                      f'<axis xyz="{axis}"/></joint>')
+    body = '<inertial><mass value="1"/><inertia ixx="0.1" iyy="0.1" izz="0.1" ixy="0" ixz="0" iyz="0"/></inertial>'
+    urdf = tmp_path / "hands.urdf"
+    urdf.write_text('<robot name="hands">' + "".join(f'<link name="{n}">{body}</link>' for n in links)
+                    + "".join(joints) + "</robot>")
+    gen = tmp_path / "_gen"
+    G.main(str(gen), str(urdf))
+    for h in glob.glob(os.path.join(HERE, "..", "pinocchio_amd", "csrc", "*.hpp")):
+        shutil.copy(h, tmp_path)
+    subprocess.run([hipcc, "-std=c++20", "--offload-arch=gfx950", "--cuda-device-only", "-fsyntax-only",
+                    "-Wno-unused-command-line-argument", str(gen / f"inst_robot_hands_{family}.hip")], check=True)
