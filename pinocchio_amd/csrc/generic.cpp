@@ -188,12 +188,12 @@ template<class S> size_t kinLane(GM g) { return (size_t)g->nlev * kGKinLvl * kTi
 
 template<class S>
 void gRnea(hipStream_t st, GM g, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> out) {
-  if (treeDynPays(false, g->nlev, sizeof(S), B) && treeRnea<S>(st, g, mc, B, q, v, a, out)) return;
+  if (treeDynPays(false, g->shape(), sizeof(S), B) && treeRnea<S>(st, g, mc, B, q, v, a, out)) return;
   RBD_G_LAUNCH(g_rnea, S, rneaLane<S>(g), B, progOf(g), mc, B, q, v, a, CView<S>{}, out);
 }
 template<class S>
 void gAba(hipStream_t st, GM g, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> tau, View<S> out) {
-  if (treeDynPays(true, g->nlev, sizeof(S), B) && treeAba<S>(st, g, mc, B, q, v, tau, out)) return;
+  if (treeDynPays(true, g->shape(), sizeof(S), B) && treeAba<S>(st, g, mc, B, q, v, tau, out)) return;
   RBD_G_LAUNCH(g_aba, S, abaLane<S>(g), B, progOf(g), mc, B, q, v, tau, CView<S>{}, out);
 }
 template<class S> void gCrba(hipStream_t st, GM g, const S* mc, int64_t B, CView<S> q, View<S> M, int upper) {

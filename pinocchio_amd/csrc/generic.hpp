@@ -36,6 +36,8 @@ struct GenericModel {
   // tables of the tree-parallel kernels; null when the numbering is not depth first
   std::unique_ptr<TreeProgram> tree;
 
+  TreeShape shape() const { return {nj - 1, nv, nlev}; }
+
   GenericModel() = default;
   GenericModel(const GenericModel&) = delete;
   GenericModel& operator=(const GenericModel&) = delete;

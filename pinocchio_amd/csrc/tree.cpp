@@ -235,13 +235,27 @@ bool treePays(TreeOp op, bool prebuilt, bool rows, int nv, int es, int64_t B) {
   return op == TreeOp::kCrba ? B * es <= 12288 : B <= 6144;
 }
 
-// The tree-parallel sweeps take a few phases per level with most lanes idle, so they win
-// until the lane-per-configuration ones fill the chip: that is later for a shallow tree.
-// us per call, run-time topology / tree-parallel: RNEA 10 levels (36 dofs) 72 / 33 at one
-// configuration, 80 / 57 at 16,384, 172 / 179 at 65,536; 40 levels (a chain) 110 / 75 at
-// 4,096, 112 / 131 at 8,192.  ABA 10 levels 224 / 45, 309 / 139, 489 / 510; 40 levels 475 /
-// 453 at 16,384; 4 levels (18 dofs) 63 / 29 at one, 118 / 118 at 65,536, FP64 243 / 286.
-bool treeDynPays(bool aba, int nlev, int es, int64_t B) { return B * es * nlev <= (aba ? 1400000 : 655360); }
+// The tree-parallel sweeps take a few phases per level with most lanes idle.  While all
+// tiles are resident (some 16,384 FP32 configurations) a call takes one tile's time; beyond,
+// time grows with the batch, and the lane-per-configuration kernels win once they fill the
+// chip: later for a shallow tree (a shorter sweep) and for one of many joints (a longer walk),
+// at once for one or two joints.  us per call, lane per configuration / tree-parallel:
+//   RNEA, 10 levels (31 joints) 76 / 32 at 1,024, 76 / 54 at 16,384, 79 / 73 at 24,576, 79 / 92
+//   at 32,768; 10 in a chain 34 / 32, 35 / 36 (24,576), FP64 45 / 33 at 8,192, 46 / 51 at 16,384;
+//   40 in a chain 108 / 72 at 4,096, 111 / 129 at 8,192; six 26 / 26 at 16,384, 26 / 28 at 24,576,
+//   FP64 30 / 29, 31 / 40; 12 at the root 32 / 25 at 32,768, 34 / 32 at 65,536, 34 / 39 at 98,304;
+//   three in a chain 20 / 20 at 1,024, 20 / 24 at 32,768; two 18 / 19 at 1,024, 19 / 30 at 65,536.
+//   ABA, 10 levels 235 / 46 at 1,024, 413 / 261 at 32,768, 447 / 383 at 49,152, 485 / 518 at
+//   65,536; 40 in a chain 465 / 240 at 8,192, 468 / 350 at 12,288, 473 / 460 at 16,384; six 81 / 65
+//   at 32,768, 88 / 85 at 49,152, 91 / 103; five 32 / 32 at 16,384, 33 / 56 at 32,768; three 25 / 26
+//   at 16,384, FP64 38 / 27 at 8,192, 38 / 40 at 16,384; six at the root 30 / 30 at 49,152, FP64
+//   35 / 32 at 32,768; two 21 / 21 at 1,024, 21 / 23 at 16,384; one 18 / 33 at 65,536.
+bool treeDynPays(bool aba, TreeShape t, int es, int64_t B) {
+  const int64_t n = B * es;
+  if (t.joints < 3) return false;
+  if (aba) return n <= (t.joints < 6 ? 65536 : 30000 * t.joints) && n * t.nlev <= 1400000;
+  return n <= 10923 * t.joints && n * t.nlev <= 655360;
+}
 
 template<class S> bool treeCrba(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, View<S> M, int upper) {
   const TProg* g = prog(m);

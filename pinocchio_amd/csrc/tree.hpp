@@ -25,13 +25,16 @@ struct TreeProgram {
 };
 TreeProgram* buildTreeProgram(int nj, const int* parents, const int* types, std::vector<int32_t>& words);
 
+struct TreeShape {
+  int joints, nv, nlev;  // the universe not counted; levels of the tree
+};
 // Whether a call is faster on the tree-parallel kernels.  prebuilt: the tree has kernels of
 // its own; rows: the output keeps a configuration's elements together (rs == 1); es: bytes
 // of a scalar.
 enum class TreeOp { kCrba, kMinv, kDeriv };
 bool treePays(TreeOp op, bool prebuilt, bool rows, int nv, int es, int64_t B);
-// RNEA and ABA of a tree without kernels of its own; nlev: levels of the tree
-bool treeDynPays(bool aba, int nlev, int es, int64_t B);
+// RNEA and ABA of a tree without kernels of its own
+bool treeDynPays(bool aba, TreeShape t, int es, int64_t B);
 
 // Each returns false, having launched nothing, when the model has no tree program or its
 // state does not fit the LDS: the caller then runs the lane-per-configuration kernels.
