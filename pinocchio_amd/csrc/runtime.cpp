@@ -239,7 +239,7 @@ void crbaInto(rbd_ctx* ctx, const rbd_model* m, int64_t B, CView<S> q, View<S> M
   const S* mc;
   if constexpr (std::is_same_v<S, float>) mc = m->mc32;
   else mc = m->mc64;
-  if (treePays(TreeOp::kCrba, m->prebuilt && m->prebuilt->crba_f32, M.rs == 1, m->nv, sizeof(S), B) &&
+  if (treePays(TreeOp::kCrba, m->gen->shape(), m->prebuilt && m->prebuilt->crba_f32, M.rs == 1, sizeof(S), B) &&
       treeCrba<S>(ctx->stream, m->gen.get(), mc, B, q, M, upper))
     return;
   if constexpr (std::is_same_v<S, float>) m->ops->crba_f32(ctx->stream, m->gen.get(), mc, B, q, M, upper);
@@ -903,8 +903,8 @@ void abaDerivCall(rbd_ctx* ctx, const rbd_model* m, int64_t B, const void* q, in
                                                                       : kTreeWsBytes / sizeof(S);
   const int64_t chunk = te ? std::min<int64_t>((B + 7) & ~int64_t(7), (wsElems / te) & ~size_t(7)) : 0;
   const size_t tneed = (size_t)nv * B + te * chunk;
-  bool tree = chunk > 0 && treePays(TreeOp::kDeriv, m->prebuilt && m->prebuilt->abad_solve_f32, vo.rs == 1, nv,
-                                    sizeof(S), B);
+  bool tree = chunk > 0 && treePays(TreeOp::kDeriv, m->gen->shape(), m->prebuilt && m->prebuilt->abad_solve_f32,
+                                    vo.rs == 1, sizeof(S), B);
   if (tree && ctx->capturing && !fixedWs && ctx->workBytes < tneed * sizeof(S)) tree = false;
   S* wU = fixedWs ? fixedWs : (S*)ctx->workspace((tree ? std::max(need, tneed) : need) * sizeof(S));
   S* wD = wU + nU;
@@ -1025,7 +1025,7 @@ int rbd_compute_minverse(rbd_ctx* ctx, const rbd_model* m, int64_t B, int dtype,
       // host outputs with gaps (padded leading dimension, batch-fastest layout) are
       // preloaded so the copy back leaves the gaps as the caller had them
       float* Mi = (float*)st.out(Minv, vo.extent * 4, (flags & RBD_LAYOUT_BATCH) || ldM != (int64_t)nv * nv);
-      if (treePays(TreeOp::kMinv, m->prebuilt && m->prebuilt->crba_f32, vo.rs == 1, nv, 4, B) &&
+      if (treePays(TreeOp::kMinv, m->gen->shape(), m->prebuilt && m->prebuilt->crba_f32, vo.rs == 1, 4, B) &&
           treeMinv<float>(ctx->stream, m->gen.get(), m->mc32, B, CView<float>{dq_, vq.rs, vq.bs},
                           View<float>{Mi, vo.rs, vo.bs})) {
         finishCall(ctx, flags, st);
@@ -1051,7 +1051,7 @@ int rbd_compute_minverse(rbd_ctx* ctx, const rbd_model* m, int64_t B, int dtype,
     Staged st{ctx, (flags & RBD_HOST_PTRS) != 0};
     const double* dq_ = (const double*)st.in(q, vq.extent * 8);
     double* Mi = (double*)st.out(Minv, vo.extent * 8, (flags & RBD_LAYOUT_BATCH) || ldM != (int64_t)nv * nv);
-    if (treePays(TreeOp::kMinv, m->prebuilt && m->prebuilt->crba_f32, vo.rs == 1, nv, 8, B) &&
+    if (treePays(TreeOp::kMinv, m->gen->shape(), m->prebuilt && m->prebuilt->crba_f32, vo.rs == 1, 8, B) &&
         treeMinv<double>(ctx->stream, m->gen.get(), m->mc64, B, CView<double>{dq_, vq.rs, vq.bs},
                          View<double>{Mi, vo.rs, vo.bs})) {
       finishCall(ctx, flags, st);

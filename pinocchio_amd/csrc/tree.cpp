@@ -210,29 +210,69 @@ const TProg* prog(GM m) { return m->tree ? m->tree->g.get() : nullptr; }
 
 }  // namespace
 
-// Measured on an MI355X, us per synchronous call, lane per configuration / tree-parallel.
-// Trees without kernels of their own: faster at every size (27 joints, CRBA 232 / 22 at one
-// configuration, 1009 / 49 at 16,384 by rows, 494 / 169 at 65,536 batch-fastest; Minv 884 /
-// 39, 2118 / 135, 2749 / 461).
-// Output by rows: 36 dofs 53 / 23 at one configuration, 1078 / 56 at 16,384, 4346 / 179 at
-// 65,536 (Minv 103 / 40, 2144 / 143, 8778 / 507; ABA derivatives 217 / 100, 4976 / 465,
-// 20586 / 1806).  Matrices of a few hundred bytes stay where they were, but for the
-// derivatives: one configuration is a few cache lines and the serial walk is short (6
-// dofs: equal up to 16,384, FP64 21 / 28 there; derivatives 64 / 58).
+// Measured on an MI355X, us per synchronous call, lane per configuration / tree-parallel;
+// FP32 unless said.
+// Trees without kernels of their own: faster at every size from five dofs up (27 joints, CRBA
+// 3996 / 130 at 65,536 by rows, 494 / 161 batch-fastest; Minv 7560 / 380, 2745 / 362; ABA
+// derivatives 18223 / 1681, 7791 / 1721; chains of 5 to 40 joints and 12 joints at the root
+// alike), but for
+//  * the smallest trees, whose serial walk is a few us, beyond the batch that one round of
+//    tiles covers.  CRBA: one joint 16 / 17 at 4,096, 16 / 21 at 65,536; a free flyer batch-
+//    fastest 24 / 20 at 32,768, 24 / 26 at 65,536, FP64 25 / 21 at 16,384, 26 / 35 at 65,536; two
+//    joints 18 / 18 at 16,384, 19 / 23 at 65,536; three 21 / 21 at 32,768, 31 / 34 at 131,072;
+//    five batch-fastest 28 / 23 at 32,768, 29 / 32 at 65,536; four at the root FP64 26 / 23 at
+//    32,768, 29 / 41 at 131,072, twelve 62 / 40, 74 / 99.  Minv: one joint 21 / 20 at 32,768,
+//    22 / 30 at 131,072; a free flyer batch-fastest 52 / 42 at 65,536, 59 / 64 at 131,072 (FP64
+//    266 / 195 at 262,144); four joints 38 / 33 at 65,536, four at the root 48 / 51 at 262,144.
+//    Derivatives: one joint 28 / 32 at 4,096, 30 / 62 at 65,536; two 39 / 40 at 8,192, 40 / 56 at
+//    32,768; three 101 / 103 at 65,536, 137 / 174 at 131,072; a free flyer batch-fastest 83 / 75 at
+//    32,768, 117 / 117, 174 / 195 at 131,072; four at the root 54 / 50 at 32,768, 59 / 72 at 65,536.
+//  * CRBA batch-fastest in FP64 beyond about 1 GiB of M (a tile writes 64 bytes of each row, the
+//    rows a whole batch apart; not traced further): 31 joints 537 / 512 at 65,536,
+//    973 / 1026 at 131,072, 1926 / 2415 at 262,144; 30 in a chain 1029 / 1028 at 131,072, 1995 /
+//    2304; 18 dofs 593 / 580 at 262,144, 1108 / 1168 at 524,288.
+// Trees with kernels of their own, output by rows: 36 dofs, CRBA 33 / 22 at one configuration,
+// 1012 / 48 at 16,384, 4369 / 157 at 65,536 (Minv 71 / 41, 2048 / 124, 8867 / 441; ABA derivatives
+// 211 / 87, 4967 / 371, 20686 / 1582).  Matrices of a few hundred bytes stay where they were, but
+// for the derivatives: one configuration is a few cache lines and the serial walk is short (6
+// dofs: equal up to 16,384, FP64 21 / 23 there; derivatives 60 / 56; of a single free flyer 42 /
+// 42 at 8,192, 75 / 66 at 32,768; of a pendulum 25 / 29 at 1,024, 26 / 45 at 65,536).
 // Batch-fastest output: where the lane-per-configuration kernels' walk is longer than the
-// phases of the tiles of a CU (36 dofs, CRBA 34 / 24 at one configuration, 34 / 33 at 4,096,
-// 34 / 45 at 8,192, FP64 38 / 31 at 1,024, 38 / 50 at 4,096; 18 dofs 22 / 22 at 1,024; Minv 75 /
-// 52 at 4,096, 79 / 84 at 8,192; 18 dofs 35 / 32, 36 / 35, 37 / 54 at 16,384; derivatives 36
-// dofs 223 / 143 at 4,096, 229 / 264 at 8,192, FP64 766 / 485 at 8,192, 934 / 1028 at 16,384; 18
-// dofs 79 / 68, 86 / 99, FP64 216 / 151, 242 / 246).  FP64 Minv was one solve launch per
-// column: 1599 / 293 at 16,384.
-bool treePays(TreeOp op, bool prebuilt, bool rows, int nv, int es, int64_t B) {
-  if (!prebuilt) return true;
-  if (op == TreeOp::kDeriv) return rows || B * 4 <= (nv < 12 ? 2048 : 5120) * es;
-  if (op == TreeOp::kMinv && es == 8) return true;
+// phases of the tiles of a CU (36 dofs, CRBA 33 / 22 at one configuration, 33 / 31 at 3,072,
+// 33 / 37 at 5,120, FP64 36 / 30 at 1,024, 36 / 47 at 3,072; 18 dofs 21 / 21 at 2,048; Minv 75 /
+// 59 at 6,144, 77 / 80 at 8,192; 18 dofs 34 / 32, 35 / 34, 36 / 46 at 12,288; derivatives 36 dofs
+// 221 / 185 at 5,120, 225 / 205 at 8,192, 229 / 258 at 10,240, FP64 856 / 566 at 10,240, 926 / 973
+// at 16,384; 18 dofs 75 / 71 at 5,120, 81 / 85 at 8,192, FP64 227 / 172 at 10,240, 235 / 254 at
+// 16,384; 7 dofs 53 / 50 at 1,024, 53 / 52 at 4,096, FP64 73 / 57 at 4,096, 87 / 88 at 16,384).
+// FP64 Minv is one solve launch per column there: 36 dofs 1611 / 298 at 16,384, 12213 / 4640 at
+// 262,144; 7 dofs 91 / 85 at 65,536, 136 / 148 at 131,072; a pendulum 23 / 22 at 32,768, 23 / 28
+// at 65,536.
+bool treePays(TreeOp op, TreeShape t, bool prebuilt, bool rows, int es, int64_t B) {
+  const int nv = t.nv;
+  const int64_t n = B * es;
+  if (!prebuilt) {
+    switch (op) {
+      case TreeOp::kCrba:
+        if (nv < 3) return nv == 2 && n <= 65536;
+        if (rows) return nv > 3 || n <= 131072;
+        if (t.joints < 3 || nv < 6 || t.nlev < 2) return n <= 131072;
+        return es == 4 || B * nv * nv <= int64_t(1) << 27;
+      case TreeOp::kMinv:
+        if (nv < 3) return n <= 131072;
+        return rows || es == 8 || (t.joints > 1 && nv > 4) || n <= 262144;
+      case TreeOp::kDeriv:
+        if (nv < 4) return nv == 3 ? n <= 262144 : nv == 2 && n <= 32768;
+        return rows || t.nlev > 1 || t.joints > 7 || n <= 131072;
+    }
+  }
+  if (op == TreeOp::kDeriv) {
+    if (t.joints < 2) return rows && nv > 1 && n > 65536;
+    return rows || B * 4 <= (nv < 12 ? 2048 : 5120) * es;
+  }
+  if (op == TreeOp::kMinv && es == 8) return (nv > 1 && rows) || nv >= 12 || n <= (nv > 1 ? 524288 : 262144);
   if (rows) return nv * nv * es > 512;
   if (nv < 12) return false;
-  return op == TreeOp::kCrba ? B * es <= 12288 : B <= 6144;
+  return op == TreeOp::kCrba ? n <= 12288 : B <= 6144;
 }
 
 // The tree-parallel sweeps take a few phases per level with most lanes idle.  While all

@@ -32,7 +32,7 @@ struct TreeShape {
 // its own; rows: the output keeps a configuration's elements together (rs == 1); es: bytes
 // of a scalar.
 enum class TreeOp { kCrba, kMinv, kDeriv };
-bool treePays(TreeOp op, bool prebuilt, bool rows, int nv, int es, int64_t B);
+bool treePays(TreeOp op, TreeShape t, bool prebuilt, bool rows, int es, int64_t B);
 // RNEA and ABA of a tree without kernels of its own
 bool treeDynPays(bool aba, TreeShape t, int es, int64_t B);
 

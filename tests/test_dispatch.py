@@ -13,7 +13,8 @@ class TreeShape(ctypes.Structure):
 
 
 PENDULUM, FREE_BODY, CHAIN2, CHAIN5 = (1, 1, 1), (1, 6, 1), (2, 2, 2), (5, 5, 5)
-CHAIN30, STAR4, HUMANOID = (30, 30, 30), (4, 4, 1), (31, 36, 10)
+CHAIN30, STAR4, HUMANOID, ARM7 = (30, 30, 30), (4, 4, 1), (31, 36, 10), (7, 7, 7)
+CRBA, MINV, DERIV = range(3)
 
 
 def rule(symbol, *args):
@@ -27,11 +28,42 @@ def dyn(aba, tree, es, B):
                 ctypes.c_int64(B))
 
 
-@pytest.mark.parametrize("tree,aba,es,B,pays", [
+def pays(op, tree, prebuilt, rows, es, B):
+    return rule("_ZN3rbd8treePaysENS_6TreeOpENS_9TreeShapeEbbil", ctypes.c_int(op), TreeShape(*tree),
+                ctypes.c_bool(prebuilt), ctypes.c_bool(rows), ctypes.c_int(es), ctypes.c_int64(B))
+
+
+@pytest.mark.parametrize("tree,aba,es,B,expect", [
     (PENDULUM, True, 4, 262144, False), (PENDULUM, False, 4, 65536, False), (FREE_BODY, True, 4, 65536, False),
     (FREE_BODY, True, 8, 16384, False), (CHAIN2, False, 4, 65536, False), (CHAIN2, True, 4, 65536, False),
     (CHAIN5, True, 4, 32768, False), (CHAIN5, False, 4, 65536, False), (STAR4, False, 4, 131072, False),
     (CHAIN5, True, 8, 8192, True), (STAR4, True, 4, 4096, True), (HUMANOID, False, 4, 16384, True),
     (HUMANOID, True, 4, 32768, True), (HUMANOID, True, 4, 65536, False), (CHAIN30, False, 4, 16384, False)])
-def test_rnea_and_aba(tree, aba, es, B, pays):
-    assert dyn(aba, tree, es, B) is pays
+def test_rnea_and_aba(tree, aba, es, B, expect):
+    assert dyn(aba, tree, es, B) is expect
+
+
+@pytest.mark.parametrize("op,tree,rows,es,B,expect", [
+    (CRBA, PENDULUM, True, 8, 262144, False), (CRBA, PENDULUM, False, 4, 65536, False),
+    (CRBA, FREE_BODY, False, 8, 65536, False), (CRBA, CHAIN2, False, 4, 262144, False),
+    (CRBA, HUMANOID, False, 8, 262144, False), (CRBA, CHAIN30, False, 8, 262144, False),
+    (CRBA, FREE_BODY, True, 4, 262144, True), (CRBA, HUMANOID, False, 4, 262144, True),
+    (CRBA, HUMANOID, True, 8, 262144, True), (CRBA, CHAIN30, False, 4, 262144, True),
+    (MINV, PENDULUM, True, 8, 262144, False), (MINV, FREE_BODY, False, 4, 131072, False),
+    (MINV, FREE_BODY, False, 8, 262144, True), (MINV, CHAIN30, False, 8, 262144, True),
+    (DERIV, PENDULUM, True, 4, 16384, False), (DERIV, CHAIN2, True, 8, 65536, False),
+    (DERIV, FREE_BODY, False, 8, 65536, False), (DERIV, STAR4, False, 4, 65536, False),
+    (DERIV, CHAIN5, False, 4, 65536, True), (DERIV, HUMANOID, False, 8, 262144, True)])
+def test_matrices_of_trees_without_kernels_of_their_own(op, tree, rows, es, B, expect):
+    assert pays(op, tree, False, rows, es, B) is expect
+
+
+@pytest.mark.parametrize("op,tree,rows,es,B,expect", [
+    (MINV, ARM7, False, 8, 262144, False), (MINV, FREE_BODY, False, 8, 262144, False),
+    (MINV, PENDULUM, True, 8, 262144, False), (MINV, ARM7, True, 8, 262144, True),
+    (MINV, HUMANOID, False, 8, 262144, True), (DERIV, PENDULUM, True, 4, 65536, False),
+    (DERIV, FREE_BODY, False, 4, 1024, False), (DERIV, FREE_BODY, True, 4, 65536, True),
+    (DERIV, HUMANOID, False, 4, 4096, True), (DERIV, HUMANOID, False, 4, 16384, False),
+    (CRBA, HUMANOID, True, 4, 1, True), (CRBA, HUMANOID, False, 4, 8192, False), (CRBA, ARM7, True, 4, 4096, False)])
+def test_matrices_of_prebuilt_trees(op, tree, rows, es, B, expect):
+    assert pays(op, tree, True, rows, es, B) is expect
