@@ -11,6 +11,15 @@
 
 namespace rbd {
 
+// The prebuilt tree factor on four waves per tile instead of one.  Batch-fastest M up to one
+// tile per CU (humanoid, 16,384: FP64 27 us of kernel, 15 on four; FP32 staged 22, 12; us per
+// call at one configuration 38 / 29).  M by rows while the rows being read are few: a lane reads
+// its own row, and the lines that four waves have in flight at once push each other out of the
+// caches (us per call, one wave / four: 36 dofs 38 / 29 at one configuration, 46 / 45 at 2,048,
+// 49 / 62 at 3,072, 60 / 81 at 4,096, 250 / 267 at 16,384, FP64 M 47 / 47 at 1,536, 47 / 51 at
+// 2,048; 18 dofs 31 / 31 at 4,096, 38 / 43 at 8,192).
+bool cholSplitPaysAt(int nv, bool rows, int64_t B) { return B <= (rows ? 65536 / nv : 16384); }
+
 namespace {
 // x <- U x: x_r += U_rc x_c over each column c in increasing order (x_c is not yet changed:
 // only columns after c write it)

@@ -138,12 +138,12 @@ void launchCrba(hipStream_t st, GM, const S* mc, int64_t B, CView<S> q, View<S> 
   else
     hipLaunchKernelGGL((k_crba<TP, S, 2>), dim3(gridFor(B)), dim3(kTile * 2), 0, st, mc, B, q, M, upper);
 }
-// four waves per tile up to one tile per CU (humanoid, 16,384: FP64 27 us of kernel, 15 on
-// four; FP32 staged 22, 12)
+// four waves per tile where that pays (cholops.cpp)
+bool cholSplitPaysAt(int nv, bool rows, int64_t B);
 template<class TP, class SIN, class SC>
 bool launchCholWaves(hipStream_t st, int64_t B, CView<SIN> M, View<SC> U, View<SC> D) {
   if constexpr (cholSplitPaysFor<TP, SIN, SC, 4>()) {
-    if (B <= 256 * kTile) {
+    if (cholSplitPaysAt(TP::T.nv, M.rs == 1, B)) {
       hipLaunchKernelGGL((k_chol_waves<TP, SIN, SC, 4>), dim3(gridFor(B)), dim3(kTile * 4), 0, st, B, M, U, D);
       return true;
     }

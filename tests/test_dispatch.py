@@ -1,6 +1,6 @@
-"""The dispatch rules that choose between the tree-parallel kernels and the lane-per-configuration
-ones: host functions of the library, no GPU.  Each row is a call whose two sides are given beside
-the rule (tree.cpp), at sizes where they differ by more than the spread of the timings."""
+"""The dispatch rules that choose between two kernels for a call: host functions of the library, no
+GPU.  Each row is a call whose two sides are given beside the rule (tree.cpp, cholops.cpp), at sizes
+where they differ by more than the spread of the timings."""
 import ctypes
 
 import pytest
@@ -67,3 +67,10 @@ def test_matrices_of_trees_without_kernels_of_their_own(op, tree, rows, es, B, e
     (CRBA, HUMANOID, True, 4, 1, True), (CRBA, HUMANOID, False, 4, 8192, False), (CRBA, ARM7, True, 4, 4096, False)])
 def test_matrices_of_prebuilt_trees(op, tree, rows, es, B, expect):
     assert pays(op, tree, True, rows, es, B) is expect
+
+
+@pytest.mark.parametrize("nv,rows,B,expect", [
+    (36, True, 1, True), (36, True, 1024, True), (36, True, 4096, False), (36, True, 16384, False),
+    (18, True, 1024, True), (18, True, 8192, False), (36, False, 16384, True), (36, False, 16385, False)])
+def test_tree_factor_on_four_waves(nv, rows, B, expect):
+    assert rule("_ZN3rbd15cholSplitPaysAtEibl", ctypes.c_int(nv), ctypes.c_bool(rows), ctypes.c_int64(B)) is expect
