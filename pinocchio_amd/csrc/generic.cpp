@@ -136,6 +136,13 @@ void* GenericModel::laneMem(size_t bytes) const {
 // ---------------------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------------------
+// Row outputs of the kinematics as runs of vectors instead of single elements: always faster
+// with placements or motions among them (31 joints, all three, elements / runs: 90 / 79 us a call at
+// 1,024 configurations, 402 / 90 at 16,384), and for the Jacobian alone in FP32 (50 / 50, 59 / 52).  A
+// small batch's FP64 Jacobian leaves faster by elements (58 / 61 at 4,096, 60 / 62 at 8,192, 80 / 69
+// at 12,288; 60 joints 95 / 103, 97 / 111, 151 / 119).
+bool kinRunsPay(bool onlyJ, int es, int64_t B) { return !onlyJ || es == 4 || B > 8192; }
+
 namespace {
 
 constexpr int64_t kGMaxGrid = 2048;        // persistent workgroups (eight per CU)
@@ -207,7 +214,7 @@ void gRneaD(hipStream_t st, GM g, const S* mc, int64_t B, CView<S> q, CView<S> v
 template<class S>
 void gKin(hipStream_t st, GM g, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> oM, View<S> vo,
           View<S> ao, View<S> J, const KinMask&) {
-  if (kinRows(oM, vo, ao, J))
+  if (kinRows(oM, vo, ao, J) && kinRunsPay(!oM.p && !vo.p, sizeof(S), B))
     RBD_G_LAUNCH(g_kin_rows, S, kinLane<S>(g), B, progOf(g), mc, B, q, v, a, oM, vo, ao, J);
   else
     RBD_G_LAUNCH(g_kin, S, kinLane<S>(g), B, progOf(g), mc, B, q, v, a, oM, vo, ao, J);

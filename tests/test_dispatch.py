@@ -1,5 +1,5 @@
 """The dispatch rules that choose between two kernels for a call: host functions of the library, no
-GPU.  Each row is a call whose two sides are given beside the rule (tree.cpp, cholops.cpp), at sizes
+GPU.  Each row is a call whose two sides are given beside the rule (tree.cpp, cholops.cpp, generic.cpp), at sizes
 where they differ by more than the spread of the timings."""
 import ctypes
 
@@ -74,3 +74,9 @@ def test_matrices_of_prebuilt_trees(op, tree, rows, es, B, expect):
     (18, True, 1024, True), (18, True, 8192, False), (36, False, 16384, True), (36, False, 16385, False)])
 def test_tree_factor_on_four_waves(nv, rows, B, expect):
     assert rule("_ZN3rbd15cholSplitPaysAtEibl", ctypes.c_int(nv), ctypes.c_bool(rows), ctypes.c_int64(B)) is expect
+
+
+@pytest.mark.parametrize("only_j,es,B,expect", [
+    (True, 8, 64, False), (True, 8, 4096, False), (True, 8, 16384, True), (True, 4, 64, True), (False, 8, 64, True)])
+def test_kinematics_rows_of_run_time_topologies(only_j, es, B, expect):
+    assert rule("_ZN3rbd11kinRunsPayEbil", ctypes.c_bool(only_j), ctypes.c_int(es), ctypes.c_int64(B)) is expect
