@@ -79,4 +79,4 @@ def test_tree_factor_on_four_waves(nv, rows, B, expect):
 @pytest.mark.parametrize("only_j,es,B,expect", [
     (True, 8, 64, False), (True, 8, 4096, False), (True, 8, 16384, True), (True, 4, 64, True), (False, 8, 64, True)])
 def test_kinematics_rows_of_run_time_topologies(only_j, es, B, expect):
-    assert rule("_ZN3rbd11kinRunsPayEbil", ctypes.c_bool(only_j), ctypes.c_int(es), ctypes.c_int64(B)) is expect
+    assert rule("_ZN3rbd10kinRunsPayEbil", ctypes.c_bool(only_j), ctypes.c_int(es), ctypes.c_int64(B)) is expect
