@@ -45,7 +45,7 @@ template<class TP, class S>
 void launchRnea(hipStream_t st, GM, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> out) {
   if constexpr (rneaSplitPaysFor<TP, S, 4>()) {
     constexpr int perCu = 160 * 1024 / (rneaWavesLdsBytes<TP, 4>() / 4 * (int)sizeof(S));
-    if (sizeof(S) == 8 || perCu >= 4 || B <= (int64_t)perCu * 256 * kTile) {
+    if ((sizeof(S) == 8 || perCu >= 4 || B <= (int64_t)perCu * 256 * kTile) && gridFits(B / kTile + 1, 4 * kTile)) {
       hipLaunchKernelGGL((k_rnea_waves<TP, S, 4>), dim3(gridFor(B)), dim3(kTile * 4), 0, st, mc, B, q, v, a, out);
       return;
     }
@@ -216,7 +216,7 @@ void launchKin(hipStream_t st, GM, const S* mc, int64_t B, CView<S> q, CView<S> 
                        want);
   };
   const bool onlyJ = !oM.p && !vo.p;
-  if (kinRows(oM, vo, ao, J)) {
+  if (kinRows(oM, vo, ao, J) && gridFits(B / kTile + 1, G * kTile)) {
     constexpr int bytes = (kinInScalars<TP>() + kinRunScalars<S, KinOut::kStaged>() * G) * (int)sizeof(S);
     if constexpr (bytes <= 160 * 1024) {
       const int64_t own = G == 1 ? perCu * 3 / 2 : !onlyJ ? perCu / 2 : sizeof(S) == 8 ? perCu * 2 : perCu;

@@ -16,6 +16,10 @@ template<class S> struct CView;
 struct GenericModel;  // run-time topology program of one model (generic.hpp)
 using GM = const GenericModel*;
 
+// A launch holds fewer than 2^32 threads (the runtime refuses more): whether `workgroups` of
+// `threads` can be one.  Asked by kernels that take more threads per configuration than one.
+bool gridFits(int64_t workgroups, int threads);
+
 template<class S>
 using LaunchVec3 = void (*)(hipStream_t, GM, const S* mc, int64_t B, CView<S> in0, CView<S> in1, CView<S> in2,
                             View<S> out);

@@ -181,15 +181,15 @@ void TreeProgram::place(const int32_t* dev) { g->tab = reinterpret_cast<const in
 TreeProgram::TreeProgram() = default;
 TreeProgram::~TreeProgram() = default;
 
+bool gridFits(int64_t workgroups, int threads) { return workgroups < (int64_t(1) << 32) / threads; }
+
 namespace {
 
 constexpr size_t kLdsMax = 160 * 1024;
 
 // grid of treeTile(): a multiple of 8 covering the tiles
-unsigned treeGrid(int64_t B) {
-  const int64_t tiles = (B + kTreeT - 1) / kTreeT;
-  return (unsigned)((tiles + 7) / 8 * 8);
-}
+int64_t treeTiles(int64_t B) { return ((B + kTreeT - 1) / kTreeT + 7) / 8 * 8; }
+unsigned treeGrid(int64_t B) { return (unsigned)treeTiles(B); }
 // dynamic LDS above the default 64 KB per workgroup needs the kernel attribute
 template<class F> bool allow(F* fn, size_t bytes) {
   if (bytes <= 64 * 1024) return true;
@@ -301,7 +301,7 @@ template<class S> bool treeCrba(hipStream_t st, GM m, const S* mc, int64_t B, CV
   const TProg* g = prog(m);
   if (!g || B <= 0) return false;
   const size_t lds = treeCrbaLds<S>(*g);
-  if (!allow(&t_crba<S>, lds)) return false;
+  if (!gridFits(treeTiles(B), (int)treeThreads(*g)) || !allow(&t_crba<S>, lds)) return false;
   hipLaunchKernelGGL((t_crba<S>), dim3(treeGrid(B)), dim3(treeThreads(*g)), lds, st, *g, mc, B, q, M, upper);
   return true;
 }
@@ -310,7 +310,7 @@ template<class S> bool treeMinv(hipStream_t st, GM m, const S* mc, int64_t B, CV
   const TProg* g = prog(m);
   if (!g || B <= 0) return false;
   const size_t lds = treeMinvLds<S>(*g);
-  if (!allow(&t_minv<S>, lds)) return false;
+  if (!gridFits(treeTiles(B), (int)treeThreads(*g)) || !allow(&t_minv<S>, lds)) return false;
   hipLaunchKernelGGL((t_minv<S>), dim3(treeGrid(B)), dim3(treeThreads(*g)), lds, st, *g, mc, B, q, X);
   return true;
 }

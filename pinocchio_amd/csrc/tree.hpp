@@ -36,8 +36,9 @@ bool treePays(TreeOp op, TreeShape t, bool prebuilt, bool rows, int es, int64_t 
 // RNEA and ABA of a tree without kernels of its own
 bool treeDynPays(bool aba, TreeShape t, int es, int64_t B);
 
-// Each returns false, having launched nothing, when the model has no tree program or its
-// state does not fit the LDS: the caller then runs the lane-per-configuration kernels.
+// Each returns false, having launched nothing, when the model has no tree program, its state
+// does not fit the LDS or the batch does not fit a launch: the caller then runs the
+// lane-per-configuration kernels.
 template<class S> bool treeCrba(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, View<S> M, int upper);
 template<class S> bool treeMinv(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, View<S> X);
 template<class S>

@@ -80,3 +80,14 @@ def test_tree_factor_on_four_waves(nv, rows, B, expect):
     (True, 8, 64, False), (True, 8, 4096, False), (True, 8, 16384, True), (True, 4, 64, True), (False, 8, 64, True)])
 def test_kinematics_rows_of_run_time_topologies(only_j, es, B, expect):
     assert rule("_ZN3rbd10kinRunsPayEbil", ctypes.c_bool(only_j), ctypes.c_int(es), ctypes.c_int64(B)) is expect
+
+
+@pytest.mark.parametrize("batch,per_tile,threads,fits", [
+    (1 << 28, 8, 128, False),          # 6 dofs, tree-parallel: two threads per dof and configuration
+    ((1 << 28) - 4096, 8, 128, True), (1 << 30, 64, 256, False),  # four waves per 64 configurations
+    ((1 << 30) - 4096, 64, 256, True), (1 << 31, 64, 64, True)])
+def test_batches_beyond_one_launch(batch, per_tile, threads, fits):
+    """A launch of 2^32 threads and more is refused; a call of that size takes the kernel with fewer
+    threads per configuration."""
+    tiles = -(-batch // per_tile)
+    assert rule("_ZN3rbd8gridFitsEli", ctypes.c_int64(tiles), ctypes.c_int(threads)) is fits

@@ -117,3 +117,16 @@ def test_run_time_topologies_beyond_the_tree_parallel_kernels(gpu_ctx, tree, B, 
     out = e.aba_derivatives(Q, *(_dev(x, layout, F64) for x in (v, tau)))
     for o, r in zip(out[:3], oracle.aba_derivatives(d, sq, sv, st)[:3]):
         assert rel_err_mats(_mats(o, layout, d.nv, idx), r).max() < 1e-9
+
+
+def test_crba_beyond_a_tree_parallel_launch(gpu_ctx):
+    """2^28 configurations by rows: 16 threads each would be a launch of 2^32, which the runtime refuses."""
+    d = M.manipulator6()
+    B, nv = 1 << 28, 6
+    e = pa.Engine(pa.Model(gpu_ctx, d, runtime_topology=True), "col")
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    q = torch.rand((B, d.nq), generator=gen, device="cuda") * 6.28 - 3.14
+    out = e.crba(q)
+    idx = np.r_[np.arange(70), np.arange(B // 2 - 5, B // 2 + 5), np.arange(B - 70, B)]
+    ref = oracle.crba(d, np.ascontiguousarray(q[idx].double().cpu().numpy().T))
+    assert rel_err_mats(_mats(out, "col", nv, idx), ref).max() < 1e-5
