@@ -897,15 +897,24 @@ void abaDerivCall(rbd_ctx* ctx, const rbd_model* m, int64_t B, const void* q, in
                                 " available (at most " + std::to_string(fixedWsElems / (nnz + 2 * nv)) +
                                 " configurations of this model)");
   // tree-parallel path: ddq, then the packed tiles of a chunk of the batch (kTreeWsBytes, or
-  // what a fixed workspace holds, bounds them); not taken in a capture for which only the
-  // other path's smaller workspace was reserved
+  // what a fixed workspace holds, bounds them)
   const size_t te = treeDerivEntries(m->gen.get()), wsElems = fixedWs ? fixedWsElems - (size_t)nv * B
                                                                       : kTreeWsBytes / sizeof(S);
-  const int64_t chunk = te ? std::min<int64_t>((B + 7) & ~int64_t(7), (wsElems / te) & ~size_t(7)) : 0;
+  auto tiles = [&](size_t elems) { return te ? (int64_t)(elems / te) & ~int64_t(7) : int64_t(0); };
+  int64_t chunk = std::min<int64_t>((B + 7) & ~int64_t(7), tiles(wsElems));
+  const bool prebuilt = m->prebuilt && m->prebuilt->abad_solve_f32;
+  bool tree = chunk > 0 && treePays(TreeOp::kDeriv, m->gen->shape(), prebuilt, vo.rs == 1, sizeof(S), B);
+  // A capture allocates nothing: its chunk is what the reserved workspace holds after ddq.  A
+  // prebuilt tree needs chunks that are worth their launches (a chunk of 1,024 humanoid
+  // configurations takes some 75 us by rows, the other path 466 for the 1,024); without kernels of
+  // its own any chunk is the better path.
+  if (const size_t own = (size_t)nv * B, held = ctx->workBytes / sizeof(S);
+      tree && ctx->capturing && !fixedWs && held < own + te * chunk) {
+    const int64_t fits = held > own ? tiles(held - own) : 0;
+    tree = !prebuilt || fits >= 1024;
+    if (fits > 0) chunk = fits;  // (else the request below is refused)
+  }
   const size_t tneed = (size_t)nv * B + te * chunk;
-  bool tree = chunk > 0 && treePays(TreeOp::kDeriv, m->gen->shape(), m->prebuilt && m->prebuilt->abad_solve_f32,
-                                    vo.rs == 1, sizeof(S), B);
-  if (tree && ctx->capturing && !fixedWs && ctx->workBytes < tneed * sizeof(S)) tree = false;
   S* wU = fixedWs ? fixedWs : (S*)ctx->workspace((tree ? std::max(need, tneed) : need) * sizeof(S));
   S* wD = wU + nU;
   S* wA = tree ? wU : wD + nD;

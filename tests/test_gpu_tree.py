@@ -137,7 +137,7 @@ def test_aba_derivatives_in_chunks(ctx):
 
 
 def test_aba_derivatives_captured_after_a_smaller_workspace(ctx):
-    """A capture for which only a smaller workspace was reserved takes the other route."""
+    """A capture whose workspace an eager call of the other route reserved (it holds all packed tiles)."""
     d = M.quadruped18()
     c = pa.Context(0)
     e = pa.Engine(pa.Model(c, d), "batch")
@@ -156,6 +156,46 @@ def test_aba_derivatives_captured_after_a_smaller_workspace(ctx):
         cap.graph.launch()
         for a, b in zip((*out, ddq), ref):
             assert ((a - b).abs().max() <= 2e-4 * b.abs().max()).item()
+
+
+def test_aba_derivatives_captured_in_the_chunks_that_fit(ctx):
+    """A capture for which only the other route's smaller workspace was reserved: the packed tiles go in
+    the chunks that it holds, bit-identical to the eager call (the other route's sums differ)."""
+    d = M.quadruped18()
+    c = pa.Context(0)
+    m = pa.Model(c, d)
+    x = [_dev(y, "batch", torch.float32) for y in (lambda t: (t[0], t[1], t[3]))(inputs(d, 20_000))]
+    pa.Engine(m, "batch").aba_derivatives(*x)  # reserves (99 + 36) scalars per configuration
+    e, B = pa.Engine(m, "col"), 9000           # wants 18 + 549, of which 4,616 configurations fit
+    rows = [y[:, :B].t().contiguous() for y in x]
+    out = [torch.empty((B, d.nv, d.nv), device="cuda") for _ in range(3)]
+    ddq = torch.empty((B, d.nv), device="cuda")
+    with c.capture() as cap:
+        e.aba_derivatives(*rows, out=out, ddq_out=ddq, async_=True)
+    ref = pa.Engine(pa.Model(ctx, d), "col").aba_derivatives(*rows)
+    for _ in range(3):
+        for o in (*out, ddq):
+            o.zero_()
+        torch.cuda.synchronize()
+        cap.graph.launch()
+        assert all(torch.equal(a, b) for a, b in zip((*out, ddq), ref))
+    cap.graph.close()
+
+
+def test_aba_derivatives_capture_refused_without_a_workspace():
+    """Without kernels of its own a tree has no other path that would allocate nothing: a capture whose
+    workspace holds not even one tile is refused as any other, and the context stays usable."""
+    d = M.random_tree(20, 7)
+    c = pa.Context(0)
+    e = pa.Engine(pa.Model(c, d), "batch")
+    x = [_dev(y, "batch", torch.float32) for y in (lambda t: (t[0], t[1], t[3]))(inputs(d, 16))]
+    one = [y[:, :1].contiguous() for y in x]
+    e.aba_derivatives(*one)
+    out = [torch.empty((d.nv * d.nv, 16), device="cuda") for _ in range(3)]
+    with pytest.raises(ValueError, match="workspace"):
+        with c.capture():
+            e.aba_derivatives(*x, out=out, async_=True)
+    e.aba_derivatives(*x, out=out)
 
 
 @pytest.mark.parametrize("dt,bar", [(torch.float32, 2e-6), (torch.float64, 1e-13)])
