@@ -898,7 +898,7 @@ void abaDerivCall(rbd_ctx* ctx, const rbd_model* m, int64_t B, const void* q, in
                                 " configurations of this model)");
   // tree-parallel path: ddq, then the packed tiles of a chunk of the batch (kTreeWsBytes, or
   // what a fixed workspace holds, bounds them)
-  const size_t te = treeDerivEntries(m->gen.get()), wsElems = fixedWs ? fixedWsElems - (size_t)nv * B
+  const size_t te = treeDerivEntries<S>(m->gen.get()), wsElems = fixedWs ? fixedWsElems - (size_t)nv * B
                                                                       : kTreeWsBytes / sizeof(S);
   auto tiles = [&](size_t elems) { return te ? (int64_t)(elems / te) & ~int64_t(7) : int64_t(0); };
   int64_t chunk = std::min<int64_t>((B + 7) & ~int64_t(7), tiles(wsElems));

@@ -342,19 +342,28 @@ template bool treeAba<float>(hipStream_t, GM, const float*, int64_t, CView<float
 template bool treeAba<double>(hipStream_t, GM, const double*, int64_t, CView<double>, CView<double>, CView<double>,
                               View<double>);
 
-size_t treeDerivEntries(GM m) {
-  const TProg* g = prog(m);
-  return g ? (size_t)treeWsEntries(*g) : 0;
+namespace {
+// segments per round of the solve: two workgroups per CU where that allows any
+template<class S> int treeSolveRounds(const TProg& g) {
+  int R = 3;
+  while (R > 1 && treeSolveLds<S>(g, R) > kLdsMax / 2) --R;
+  return R;
 }
+}  // namespace
+template<class S> size_t treeDerivEntries(GM m) {
+  const TProg* g = prog(m);
+  if (!g || treeRneadLds<S>(*g) > kLdsMax || treeSolveLds<S>(*g, treeSolveRounds<S>(*g)) > kLdsMax) return 0;
+  return (size_t)treeWsEntries(*g);
+}
+template size_t treeDerivEntries<float>(GM);
+template size_t treeDerivEntries<double>(GM);
 
 template<class S>
 bool treeAbaDeriv(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> Xq,
                   View<S> Xv, View<S> Minv, S* ws) {
   const TProg* g = prog(m);
   if (!g || B <= 0) return false;
-  // segments per round of the solve: two workgroups per CU where that allows any
-  int R = 3;
-  while (R > 1 && treeSolveLds<S>(*g, R) > kLdsMax / 2) --R;
+  const int R = treeSolveRounds<S>(*g);
   const size_t l1 = treeRneadLds<S>(*g), l2 = treeSolveLds<S>(*g, R);
   if (!allow(&t_rnead<S>, l1) || !allow(&t_dsolve<S>, l2)) return false;
   const unsigned grid = treeGrid(B);

@@ -46,9 +46,10 @@ bool treeRnea(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, CView<S>
 template<class S>
 bool treeAba(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> tau, View<S> ddq);
 
-// RNEA derivatives at a and the ABA-derivative solve; ws: treeDerivEntries(m) scalars per
-// configuration, the batch rounded up to a multiple of 8.
-size_t treeDerivEntries(GM m);
+// RNEA derivatives at a and the ABA-derivative solve; ws: treeDerivEntries<S>(m) scalars per
+// configuration, the batch rounded up to a multiple of 8.  0: no tree program, or its state does
+// not fit the LDS.
+template<class S> size_t treeDerivEntries(GM m);
 template<class S>
 bool treeAbaDeriv(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, CView<S> v, CView<S> a, View<S> Xq,
                   View<S> Xv, View<S> Minv, S* ws);

@@ -130,3 +130,23 @@ def test_crba_beyond_a_tree_parallel_launch(gpu_ctx):
     idx = np.r_[np.arange(70), np.arange(B // 2 - 5, B // 2 + 5), np.arange(B - 70, B)]
     ref = oracle.crba(d, np.ascontiguousarray(q[idx].double().cpu().numpy().T))
     assert rel_err_mats(_mats(out, "col", nv, idx), ref).max() < 1e-5
+
+
+def test_aba_derivatives_beyond_the_lds_take_no_tree_workspace():
+    """60 joints in FP64, whose packed path does not fit the LDS: the call allocates what the other path
+    needs, the factor and ddq (43 MB here; the packed tiles would be 128 MiB)."""
+    d, B = M.random_tree(60, 5), 8192
+    c = pa.Context(0)
+    m = pa.Model(c, d, runtime_topology=True)
+    e = pa.Engine(m, "batch")
+    x = [_dev(y, "batch", F64) for y in (lambda t: (t[0], t[1], t[3]))(inputs(d, B))]
+    out = [torch.empty((d.nv * d.nv, B), dtype=F64, device="cuda") for _ in range(3)]
+    ddq = torch.empty((d.nv, B), dtype=F64, device="cuda")
+    e.aba_derivatives(*(y[:, :64].contiguous() for y in x))  # lane memory of the kernels, tables
+    e.aba(*x, out=ddq)
+    e.rnea_derivatives(x[0], x[1], x[2])
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    e.aba_derivatives(*x, out=out, ddq_out=ddq)
+    nnz = len(m.cholesky_pattern()[0])
+    assert free - torch.cuda.mem_get_info()[0] <= (nnz + 2 * d.nv) * B * 8 + (8 << 20)
