@@ -367,7 +367,12 @@ bool treeAbaDeriv(hipStream_t st, GM m, const S* mc, int64_t B, CView<S> q, CVie
   const size_t l1 = treeRneadLds<S>(*g), l2 = treeSolveLds<S>(*g, R);
   if (!allow(&t_rnead<S>, l1) || !allow(&t_dsolve<S>, l2)) return false;
   const unsigned grid = treeGrid(B);
-  const unsigned y = grid <= 168 ? 3 : 1;
+  // Three workgroups per tile while they find places of their own: two per CU, or one where the
+  // solve takes more than half of the LDS (us per call, one / three: 36 dofs 98 / 88 at one
+  // configuration, 104 / 97 at 1,344, 109 / 113 at 1,408; FP64, one per CU, 133 / 113 at 512,
+  // 145 / 128 at 768, 148 / 149 at 1,024, 150 / 171 at 1,344; 18 dofs FP64, two per CU, 66 / 62 at 1,344,
+  // 66 / 69 at 1,408; 30 in a chain FP64 220 / 218 at 768, 227 / 239 at 1,024).
+  const unsigned y = grid <= (l2 <= kLdsMax / 2 ? 168 : 96) ? 3 : 1;
   hipLaunchKernelGGL((t_rnead<S>), dim3(grid), dim3(treeThreads(*g)), l1, st, *g, mc, B, q, v, a, ws);
   hipLaunchKernelGGL((t_dsolve<S>), dim3(grid, y), dim3(treeThreads(*g)), l2, st, *g, B, (const S*)ws, Xq, Xv, Minv, R);
   return true;
