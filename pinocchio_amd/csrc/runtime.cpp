@@ -1024,11 +1024,6 @@ int rbd_compute_minverse(rbd_ctx* ctx, const rbd_model* m, int64_t B, int dtype,
     if (!m->compact || !m->ops->crba_f32 || !m->ops->abad_solve_f32)
       throw Error(RBD_EUNSUPPORTED, "computeMinverse: no kernels for this topology");
     const int nv = m->nv, nnz = m->ops->nnzU;
-    // an eager call on the tree-parallel kernel, which needs no workspace, reserves the other path's:
-    // a capture of the same batch in the other layout or type may take that
-    auto reserve = [&](size_t bytes) {
-      if (!ctx->capturing) (void)ctx->workspace(bytes);
-    };
     if (dtype == RBD_F32) {
       auto vq = argView<float>(m->nq, B, ldq, flags, "q");
       auto vo = argView<float>(nv * nv, B, ldM, flags, "Minv");
@@ -1039,8 +1034,6 @@ int rbd_compute_minverse(rbd_ctx* ctx, const rbd_model* m, int64_t B, int dtype,
       // host outputs with gaps (padded leading dimension, batch-fastest layout) are
       // preloaded so the copy back leaves the gaps as the caller had them
       float* Mi = (float*)st.out(Minv, vo.extent * 4, (flags & RBD_LAYOUT_BATCH) || ldM != (int64_t)nv * nv);
-      const size_t nU = (size_t)(nnz > 0 ? nnz : 1) * B, nD = (size_t)nv * B;
-      reserve((nU + nD) * 4);
       if (treePays(TreeOp::kMinv, m->gen->shape(), m->prebuilt && m->prebuilt->crba_f32, vo.rs == 1, 4, B) &&
           treeMinv<float>(ctx->stream, m->gen.get(), m->mc32, B, CView<float>{dq_, vq.rs, vq.bs},
                           View<float>{Mi, vo.rs, vo.bs})) {
@@ -1049,6 +1042,7 @@ int rbd_compute_minverse(rbd_ctx* ctx, const rbd_model* m, int64_t B, int dtype,
       }
       // M into the output buffer, its FP32 tree factor into the workspace, then the unit
       // right-hand sides of the solve overwrite M with its inverse
+      const size_t nU = (size_t)(nnz > 0 ? nnz : 1) * B, nD = (size_t)nv * B;
       float* wU = (float*)ctx->workspace((nU + nD) * 4);
       float* wD = wU + nU;
       const View<float> vM{Mi, vo.rs, vo.bs};
@@ -1058,6 +1052,7 @@ int rbd_compute_minverse(rbd_ctx* ctx, const rbd_model* m, int64_t B, int dtype,
       finishCall(ctx, flags, st);
       return;
     }
+    // FP64: FP64 CRBA and tree factor, then one solve per unit column
     auto vq = argView<double>(m->nq, B, ldq, flags, "q");
     auto vo = argView<double>(nv * nv, B, ldM, flags, "Minv");
     if (B == 0) return;
@@ -1065,16 +1060,13 @@ int rbd_compute_minverse(rbd_ctx* ctx, const rbd_model* m, int64_t B, int dtype,
     Staged st{ctx, (flags & RBD_HOST_PTRS) != 0};
     const double* dq_ = (const double*)st.in(q, vq.extent * 8);
     double* Mi = (double*)st.out(Minv, vo.extent * 8, (flags & RBD_LAYOUT_BATCH) || ldM != (int64_t)nv * nv);
-    const size_t nU = (size_t)(nnz > 0 ? nnz : 1) * B, nD = (size_t)nv * B;
-    reserve((nU + nD) * 8);
     if (treePays(TreeOp::kMinv, m->gen->shape(), m->prebuilt && m->prebuilt->crba_f32, vo.rs == 1, 8, B) &&
         treeMinv<double>(ctx->stream, m->gen.get(), m->mc64, B, CView<double>{dq_, vq.rs, vq.bs},
                          View<double>{Mi, vo.rs, vo.bs})) {
       finishCall(ctx, flags, st);
       return;
     }
-    // FP64 CRBA and tree factor, then one solve per unit column: batch-fastest matrices of fewer than
-    // 12 dofs beyond the tree-parallel kernel's batch, or a state that does not fit its LDS
+    const size_t nU = (size_t)(nnz > 0 ? nnz : 1) * B, nD = (size_t)nv * B;
     double* wU = (double*)ctx->workspace((nU + nD) * 8);
     double* wD = wU + nU;
     m->ops->crba_f64(ctx->stream, m->gen.get(), m->mc64, B, CView<double>{dq_, vq.rs, vq.bs}, View<double>{Mi, vo.rs, vo.bs}, 0);

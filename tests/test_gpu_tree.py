@@ -198,27 +198,6 @@ def test_aba_derivatives_capture_refused_without_a_workspace():
     e.aba_derivatives(*x, out=out)
 
 
-def test_minverse_captured_in_the_other_layout():
-    """An eager call by rows (tree-parallel, no workspace), then a capture of the same batch
-    batch-fastest, on kernels that need one."""
-    d, B = M.quadruped18(), 9001
-    c = pa.Context(0)
-    m = pa.Model(c, d)
-    q = _dev(inputs(d, B)[0], "col", torch.float32)
-    pa.Engine(m, "col").compute_minverse(q)
-    e, Q = pa.Engine(m, "batch"), q.t().contiguous()
-    out = torch.empty((d.nv * d.nv, B), device="cuda")
-    with c.capture() as cap:
-        e.compute_minverse(Q, out=out, async_=True)
-    ref = e.compute_minverse(Q)
-    for _ in range(3):
-        out.zero_()
-        torch.cuda.synchronize()
-        cap.graph.launch()
-        assert torch.equal(out, ref)
-    cap.graph.close()
-
-
 @pytest.mark.parametrize("dt,bar", [(torch.float32, 2e-6), (torch.float64, 1e-13)])
 @pytest.mark.parametrize("pad", [0, 1, 2, 4])
 def test_kinematics_rows(ctx, dt, bar, pad):
