@@ -20,7 +20,7 @@ template<class TP> constexpr int kinLdsRows() { return TP::T.nq + 2 * TP::T.nv; 
 // N consecutive scalars in vectors of 16 (placements) or two scalars (motions, columns):
 // with one configuration per row a lane's outputs are runs in its own row, a lane apart by
 // the row length.  Ordinary stores, so that the L2 completes a line from the runs of
-// neighbouring joints: one nontemporal scalar at a time took 952 us where this took 43
+// neighbouring joints: one nontemporal scalar at a time took 952 us where this took 47
 // (humanoid, placements and motions of 30,011 rows, 86 MB; staged on four waves, below, 31:
 // 2.8 TB/s).
 template<int N, class S> __device__ __forceinline__ void putRun(S* dst, const S* x) {

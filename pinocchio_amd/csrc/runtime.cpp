@@ -863,8 +863,8 @@ void rneaDerivCall(rbd_ctx* ctx, const rbd_model* m, int64_t B, const void* q, i
 }
 
 // ABA (ddq), RNEA derivatives at a = ddq (dtau_dq, dtau_dv, M into the outputs), the tree
-// factor of M, then Minv and -Minv dtau in place.  FP32: the prebuilt kernels where the
-// topology has them; FP64: the run-time-topology kernels.
+// factor of M, then Minv and -Minv dtau in place; after ABA the tree-parallel pair on packed
+// tiles where treePays says so.
 // fixedWs: a workspace of fixedWsElems scalars to use instead of the context's (which
 // grows by allocation); the call then allocates nothing
 template<class S>
@@ -1052,7 +1052,6 @@ int rbd_compute_minverse(rbd_ctx* ctx, const rbd_model* m, int64_t B, int dtype,
       finishCall(ctx, flags, st);
       return;
     }
-    // FP64: FP64 CRBA and tree factor, then one solve per unit column
     auto vq = argView<double>(m->nq, B, ldq, flags, "q");
     auto vo = argView<double>(nv * nv, B, ldM, flags, "Minv");
     if (B == 0) return;
@@ -1066,6 +1065,8 @@ int rbd_compute_minverse(rbd_ctx* ctx, const rbd_model* m, int64_t B, int dtype,
       finishCall(ctx, flags, st);
       return;
     }
+    // FP64 CRBA and tree factor, then one solve per unit column: batch-fastest matrices of fewer than
+    // 12 dofs beyond the tree-parallel kernel's batch, or a state that does not fit its LDS
     const size_t nU = (size_t)(nnz > 0 ? nnz : 1) * B, nD = (size_t)nv * B;
     double* wU = (double*)ctx->workspace((nU + nD) * 8);
     double* wD = wU + nU;
